@@ -12,6 +12,7 @@
 #include <type_traits>
 
 #include "rbfx_ell_common.h"
+#include "rbfx_ell_local.h"
 #include "rbfx_host_internal.h"
 
 namespace {
@@ -413,15 +414,9 @@ void rbfx_ell_destroy(rbfx_ell* e) {
     delete e;
 }
 
-int rbfx_ell_build_local(rbfx_ell* e, int32_t tile_rows, int32_t max_nodes) {
-    if (!e) return RBFX_E_INVALID;
+// The tile tables built on the host: stencils too wide, or lists too long, for the device build.
+static int local_tables_host(rbfx_ell* e, int tile_rows, int max_nodes, LocalTables* T) {
     rbfx_ctx* ctx = e->ctx;
-    if (tile_rows != 32 && tile_rows != 64 && tile_rows != 128)
-        return rbfx_fail(ctx, RBFX_E_INVALID, "ell_build_local: tile_rows %d not 32, 64 or 128", tile_rows);
-    if (max_nodes < 0 || (max_nodes > 0 && max_nodes < e->width))
-        return rbfx_fail(ctx, RBFX_E_INVALID, "ell_build_local: max_nodes %d below the stencil width %d", max_nodes,
-                         e->width);
-    RBFX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     const size_t entries = (size_t)e->n_pad * e->width;
     std::vector<int32_t> idx(entries);
     RBFX_HIP_CHECK(ctx, hipMemcpyAsync(idx.data(), e->idx_t, entries * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -432,9 +427,6 @@ int rbfx_ell_build_local(rbfx_ell* e, int32_t tile_rows, int32_t max_nodes) {
                                               pos, off, nodes, lidx);
     if (k_max < 0)
         return rbfx_fail(ctx, RBFX_E_TOO_LARGE, "ell_build_local: a tile of %d rows has more than 65535 distinct nodes", tile_rows);
-    int lds_attr = 0;
-    if (hipDeviceGetAttribute(&lds_attr, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device) != hipSuccess || lds_attr <= 0)
-        lds_attr = 64 * 1024;
     int32_t *d_pos = nullptr, *d_off = nullptr, *d_nodes = nullptr;
     uint16_t* d_lidx = nullptr;
     hipError_t err;
@@ -459,14 +451,40 @@ int rbfx_ell_build_local(rbfx_ell* e, int32_t tile_rows, int32_t max_nodes) {
         drop();
         return rbfx_fail(ctx, RBFX_E_HIP, "ell_build_local: %s", hipGetErrorString(err));
     }
+    T->pos = d_pos;
+    T->off = d_off;
+    T->nodes = d_nodes;
+    T->idx = d_lidx;
+    T->n_tiles = (int)pos.size() - 1;
+    T->k_max = k_max;
+    return RBFX_OK;
+}
+
+int rbfx_ell_build_local(rbfx_ell* e, int32_t tile_rows, int32_t max_nodes) {
+    if (!e) return RBFX_E_INVALID;
+    rbfx_ctx* ctx = e->ctx;
+    if (tile_rows != 32 && tile_rows != 64 && tile_rows != 128)
+        return rbfx_fail(ctx, RBFX_E_INVALID, "ell_build_local: tile_rows %d not 32, 64 or 128", tile_rows);
+    if (max_nodes < 0 || (max_nodes > 0 && max_nodes < e->width))
+        return rbfx_fail(ctx, RBFX_E_INVALID, "ell_build_local: max_nodes %d below the stencil width %d", max_nodes,
+                         e->width);
+    RBFX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    int lds_attr = 0;
+    if (hipDeviceGetAttribute(&lds_attr, hipDeviceAttributeMaxSharedMemoryPerBlock, ctx->device) != hipSuccess || lds_attr <= 0)
+        lds_attr = 64 * 1024;
+    LocalTables T;
+    int rc = RBFX_OK;
+    if (!rbfx_local_tables_device(e, tile_rows, max_nodes, (size_t)lds_attr, &T, &rc))
+        rc = local_tables_host(e, tile_rows, max_nodes, &T);
+    if (rc) return rc;
     free_local(e);
-    e->loc_pos = d_pos;
-    e->n_ltiles = (int)pos.size() - 1;
-    e->loc_off = d_off;
-    e->loc_nodes = d_nodes;
-    e->loc_idx = d_lidx;
+    e->loc_pos = T.pos;
+    e->n_ltiles = T.n_tiles;
+    e->loc_off = T.off;
+    e->loc_nodes = T.nodes;
+    e->loc_idx = T.idx;
     e->lt = tile_rows;
-    e->k_max = k_max;
+    e->k_max = T.k_max;
     e->lds_limit = lds_attr;
     e->layout_version++;
     return RBFX_OK;

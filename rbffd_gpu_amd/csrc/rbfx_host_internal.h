@@ -5,7 +5,8 @@
 
 #include "rbfx.h"
 
-// Local-index tables for LDS-staged gathers, built on the host from an operator set's index
+// Local-index tables for LDS-staged gathers, built on the host (for the sets the device build of
+// rbfx_ell_local.hip does not take) from an operator set's index
 // array in its device layout (tiles of tile_layout rows, slot-major inside a tile, stencil
 // width `width`; the first n_rows positions are real). Positions are cut greedily into
 // tiles of at most lt consecutive positions whose distinct neighbour nodes number at most

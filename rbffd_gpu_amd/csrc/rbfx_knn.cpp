@@ -409,8 +409,9 @@ int rbfx_build_local_tables(const int32_t* idx_layout, int n_rows, int n_pad, in
             while (p < p_hi && p - start < lt) {
                 for (int j = 0; j < width; j++) row[(size_t)j] = idx_layout[entry(p, j)];
                 std::sort(row.begin(), row.end());
+                const auto row_end = std::unique(row.begin(), row.end());  // pad slots repeat the centre
                 merged.clear();
-                std::set_union(u.begin(), u.end(), row.begin(), row.end(), std::back_inserter(merged));
+                std::set_union(u.begin(), u.end(), row.begin(), row_end, std::back_inserter(merged));
                 if (cap > 0 && p > start && (int)merged.size() > cap) break;
                 u.swap(merged);
                 p++;
