@@ -18,9 +18,11 @@
 // component), with identity rows elsewhere. The factor of -eta L is computed once and applied
 // to the three components. The dependencies of the factorization and of both sweeps follow
 // the stencil graph; rows are grouped into dependency levels on the host (a row's level is one
-// more than the deepest of the rows it reads), and one workgroup runs the levels in order with
-// a barrier between levels. Every row accumulates in the reference's order, without fused
-// multiply-adds, so the factor and the sweeps match the CPU restatement bit for bit.
+// more than the deepest of the rows it reads). The factorization runs them on one workgroup with a
+// barrier between levels; each sweep runs the three components on a workgroup each, its waves
+// handing the levels on through a counter in LDS. Every row accumulates in the reference's
+// order, without fused multiply-adds, so the factor and the sweeps match the CPU restatement bit
+// for bit.
 //
 // GMRES. Arnoldi with classical Gram-Schmidt applied twice (each pass one multi-dot kernel over
 // the basis and one multi-axpy), Givens rotations on the host. The stopping test is the
@@ -36,12 +38,15 @@ namespace {
 
 constexpr int FACTOR_THREADS = 1024;
 constexpr int FACTOR_WAVES = FACTOR_THREADS / 64;
-constexpr int SWEEP_THREADS = 512;      // a level holds a few dozen rows, up to about a hundred
-constexpr int SWEEP_CH = 32;            // entries of a row on one side of the diagonal, n <= 33
-constexpr int SWEEP_CH_MAX = 64;        // the same, n <= 64
-constexpr int SWEEP_EPL = 2;            // entries per lane: a row takes CH / 2 lanes
-__host__ __device__ constexpr int sweep_slots(int ch) { return SWEEP_THREADS / (ch / SWEEP_EPL); }
-constexpr int SWEEP_LDS_LEVELS = 8192;  // level offsets kept in LDS up to this many levels
+// A sweep's variants hold rows of up to 32, 40, 48 or 64 entries on one side of the diagonal in
+// registers: 12 waves of at most 168 VGPRs for the first, 8 of at most 256 for the others.
+constexpr int sweep_variant(int blks) { return blks <= 4 ? 4 : blks <= 7 ? blks : 8; }
+__host__ __device__ constexpr int sweep_waves(int nb) { return nb <= 4 ? 12 : 8; }
+constexpr int SWEEP_ROWS = 64;     // rows of a chunk, one per lane
+constexpr int SWEEP_BLK = 8;       // entries whose products a wave forms together
+constexpr int SWEEP_MAX_BLKS = 8;  // up to 64 entries of a row on one side of the diagonal
+constexpr int SWEEP_RING = 16384;  // solved values kept in LDS: the last 16384 tasks
+constexpr int SWEEP_ZERO = SWEEP_RING, SWEEP_ONE = SWEEP_RING + 1;  // LDS places holding 0 and 1
 constexpr int FACTOR_MAX_WIDTH = 64;  // one lane per stencil entry in the factorization
 constexpr int FACTOR_CHUNK = 8;       // L entries whose U rows a wave loads at once
 constexpr int DOT_THREADS = 256;
@@ -247,140 +252,226 @@ __global__ void __launch_bounds__(FACTOR_THREADS) ilu0_factor_kernel(const int32
     }
 }
 
-// One triangular sweep of the factor over the three velocity blocks, level by level. Task t
-// (levels in order) is row rows[t] with its entries packed at [pk_off[t], pk_off[t+1]): the
-// strictly lower entries for the forward sweep, the strictly upper ones (and the diagonal
-// pk_diag[t]) for the backward sweep, columns ascending, at most CH of them. A level holds at
-// most sweep_slots(CH) rows (the host splits larger ones) and each row takes a slot of CH / 2
-// lanes: lane l loads entries l and l + CH / 2, gathers the three components at their
-// columns and writes the products L_rq v_c[col_q] to LDS; lanes 0..2 of the slot then subtract
-// them from v_c[r] one after the other in column order (entries past the row's end hold +0,
-// and s - (+0) == s for every s), so each component accumulates exactly as the sequential
-// sweep does, and finally (UPPER) divide by U_rr.
+// One triangular sweep of the factor over one velocity block (blockIdx.x: u, v or w; the three do
+// not depend on each other and run on a CU each).
 //
-// Only the gathers depend on the previous level. A task's loads are spread over the two levels
-// before its own: two levels ahead its row and entry range (locate), one level ahead its
-// columns, values, own values and U_rr (load_entries), each issued after the current level's
-// gathers and read only a level later, so the wait on memory a level pays is for its gathers.
-// The level body has no loop (levels are split to fit the slots, CH covers the widest row),
-// which keeps the compiler's memory-counter waits close to exact. Lanes past a row's end read
-// its first entry (one address for all of them; the packed arrays carry CH zero entries past
-// their end); a slot without a row reads nothing but task 0's place, which keeps those loads
-// unconditional, and skips its entries, gathers and store.
-template <typename T, int EPL>
-struct SweepTask {
-    int t;   // task index, -1: none
-    int tt;  // t, or 0 for an empty slot
-    int r, a, e;
-    int pc[EPL];
-    T pv[EPL];
-    T s, dg;  // lanes 0..2: the row's own value of component l (written only by this task), U_rr
+// The rows of a level are cut into chunks of at most SWEEP_ROWS, chunks are numbered in level
+// order, and the workgroup's waves take them in turn: one row per lane, its entries (columns
+// ascending, at most 8 * NB of them) in registers. A row's sum has to run in column order, but its
+// products do not depend on each other, and most of its entries were solved long before the level
+// above. So while the waves before it still work, a wave forms the products of a block of 8 entries
+// as soon as the chunks they come from are done (need[b]), and, forward, where the latest solved
+// entries come last, subtracts them. On the critical path of a level stay the count of finished
+// chunks seen in LDS, the reads of the last block's values, the rest of the sum and (backward) the
+// division. There is no barrier, and a chunk's loads are issued when the wave's chunk before is
+// done, 11 (7) chunks ahead.
+//
+// Solved values stay in LDS for SWEEP_RING tasks (ring; the place of task t is t mod SWEEP_RING):
+// an entry's pk_idx is its value's place there, or, when more than SWEEP_RING tasks lie between,
+// ~row: those products are formed from memory when the entries arrive, and the entry then
+// multiplies the ring's constant 1. Pads are 0 times the ring's constant 0: s - (+0) = s for every s.
+//
+// Order. Only the wave of chunk *s_done writes to the ring, and then raises the count to its
+// successor; a wave that reads count d therefore reads values of tasks before chunk d, and finds
+// none overwritten, as pk_idx keeps to the last SWEEP_RING tasks before its own chunk. LDS operations
+// of a wave execute in the order they were issued. Values read from memory were stored at least
+// SWEEP_RING / SWEEP_ROWS chunks before, by this CU, and a wave has waited for its store by the time
+// it works on its next chunk. Every wait ends: the wave of chunk *s_done waits for no one, and all
+// waves of the workgroup are resident.
+//
+// Bound: the latency of that chain, measured in cycles per chunk forward / backward: count seen 155 /
+// 139, reads, products and sum 268 / 572 (an FP64 add takes 9.5, a division 81, a read of 8 scattered
+// values about 200), value and count written 76. N = 40962, n = 31 (1736 / 1755 chunks): 0.45 / 0.60
+// ms. One workgroup for the three components, products handed over through LDS and a barrier per 32
+// rows, took 1.83 / 2.01 ms; this kernel with scalar loads of the entries (64 per lane and chunk, the
+// CU's load rate) 0.57 / 0.63, with the final block read ahead of the count 0.70 / 0.80, with
+// 4-entry blocks 0.96 / 1.12.
+struct SweepChunk {
+    int t0, nr;            // first task, rows
+    int base;              // first packed entry
+    int nblk;              // blocks of 8 entries; bit 8: some entries are older than the ring
+    int need[SWEEP_MAX_BLKS];  // chunks that must be done before block b's products
+    int unused[4];
 };
 
-template <typename T, bool UPPER, bool LDS_OFF, int CH>
-__global__ void __launch_bounds__(SWEEP_THREADS) ilu0_sweep_kernel(const int32_t* __restrict__ rows,
-                                                                   const int32_t* __restrict__ off, int n_lev,
-                                                                   const int32_t* __restrict__ pk_off,
-                                                                   const int32_t* __restrict__ pk_col,
-                                                                   const T* __restrict__ pk_val,
-                                                                   const T* __restrict__ pk_diag, int N, T* v) {
-    constexpr int EPL = SWEEP_EPL, SL = CH / EPL, NS = sweep_slots(CH);
-    // a slot's three rows of products, padded so that the twelve summing lanes of a wave fall
-    // in different banks and each row starts on 16 bytes
-    constexpr int PS = (CH * (int)sizeof(T) + 16) / (int)sizeof(T);
-    __shared__ int s_off[LDS_OFF ? SWEEP_LDS_LEVELS + 1 : 1];
-    __shared__ __align__(16) T s_prod[NS][3][PS];
-    if (LDS_OFF)
-        for (int i = threadIdx.x; i <= n_lev; i += blockDim.x) s_off[i] = off[i];
+template <typename T, bool UPPER, int NB>
+__global__ void __launch_bounds__(64 * sweep_waves(NB)) ilu0_sweep_kernel(const SweepChunk* __restrict__ chunks, int n_chunks,
+                                                                     const int32_t* __restrict__ rows,
+                                                                     const int32_t* __restrict__ pk_idx,
+                                                                     const T* __restrict__ pk_val,
+                                                                     const T* __restrict__ pk_diag, int N, T* v_all) {
+    constexpr int WAVES = sweep_waves(NB), PER16 = 16 / (int)sizeof(T);
+    constexpr int YB = !UPPER && NB <= 6 ? 2 : 1;  // blocks of values read at once
+    extern __shared__ __align__(16) unsigned char smem[];
+    T* ring = reinterpret_cast<T*>(smem);
+    int* s_done = reinterpret_cast<int*>(ring + SWEEP_RING + 2);
+    T* v = v_all + (size_t)blockIdx.x * N;
+    const int lane = threadIdx.x % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    if (threadIdx.x == 0) {
+        ring[SWEEP_ZERO] = T(0);
+        ring[SWEEP_ONE] = T(1);
+        *s_done = 0;
+    }
     __syncthreads();
-    const int slot = (int)threadIdx.x / SL, l = (int)threadIdx.x % SL;
-    const int lc = l < 3 ? l : 2;  // lanes past 2 load a value they do not use
-    T(*P)[PS] = s_prod[slot];
-    auto level_start = [&](int lv) {
-        lv = lv < n_lev ? lv : n_lev;
-        return LDS_OFF ? s_off[lv] : off[lv];
+    auto done = [&] {
+        const int d = __hip_atomic_load(s_done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        asm volatile("" ::: "memory");  // the ring is read after the count
+        return __builtin_amdgcn_readfirstlane(d);
     };
-    auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    };
-    auto locate = [&](SweepTask<T, EPL>& X, int lev) {
-        const int t = level_start(lev) + slot;
-        const bool ok = t < level_start(lev + 1);
-        X.t = ok ? t : -1;
-        X.tt = ok ? t : 0;
-        X.r = rows[X.tt];
-        X.a = pk_off[X.tt];
-        X.e = pk_off[X.tt + 1];
-    };
-    auto load_entries = [&](SweepTask<T, EPL>& X) {
-        const int len = X.e - X.a;
-        if (X.t >= 0) {
+    // the next chunk's description and row are loaded with this chunk's entries
+    SweepChunk next_C = chunks[min(wave, n_chunks - 1)];
+    int next_r = rows[next_C.t0 + min(lane, next_C.nr - 1)];
+    for (int c = wave; c < n_chunks; c += WAVES) {
+        const SweepChunk C = next_C;
+        const int r = next_r;
+        next_C = chunks[min(c + WAVES, n_chunks - 1)];
+        const int nblk = C.nblk & 0xff;
+        const int l = lane < C.nr ? lane : C.nr - 1;  // lanes past the last row repeat it
+        int id[NB * SWEEP_BLK];
+        T p[NB * SWEEP_BLK];  // the factor's entries, then their products
 #pragma unroll
-            for (int j = 0; j < EPL; j++) {
-                const int k = l + j * SL;
-                X.pc[j] = pk_col[X.a + (k < len ? k : 0)];
-                X.pv[j] = pk_val[X.a + (k < len ? k : 0)];
+        for (int b = 0; b < NB; b++)
+            if (UPPER ? b < nblk : b >= NB - nblk) {
+                const size_t at = (size_t)C.base + (UPPER ? b : b - (NB - nblk)) * SWEEP_BLK * C.nr;
+#pragma unroll
+                for (int e = 0; e < SWEEP_BLK; e += 4) {
+                    int i4[4];
+                    load_pack<int, 4>(pk_idx + at + e * C.nr + 4 * l, i4);
+#pragma unroll
+                    for (int q = 0; q < 4; q++) id[b * SWEEP_BLK + e + q] = i4[q];
+                }
+#pragma unroll
+                for (int e = 0; e < SWEEP_BLK; e += PER16) {
+                    T v16[PER16];
+                    load_pack<T, PER16>(pk_val + at + e * C.nr + PER16 * l, v16);
+#pragma unroll
+                    for (int q = 0; q < PER16; q++) p[b * SWEEP_BLK + e + q] = v16[q];
+                }
             }
-            X.s = v[(size_t)lc * N + X.r];
-            if (UPPER) X.dg = pk_diag[X.t];
+        T s = v[r];  // written by this task only
+        const T dg = UPPER ? pk_diag[C.t0 + l] : T(1);
+        next_r = rows[next_C.t0 + min(lane, next_C.nr - 1)];
+        if (C.nblk >> 8) {
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+                if (UPPER ? b < nblk : b >= NB - nblk) {
+                    T y[SWEEP_BLK];
+#pragma unroll
+                    for (int e = 0; e < SWEEP_BLK; e++) {
+                        const int k = id[b * SWEEP_BLK + e];
+                        y[e] = __hip_atomic_load(v + (k < 0 ? ~k : r), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    }
+#pragma unroll
+                    for (int e = 0; e < SWEEP_BLK; e++) {
+                        int& k = id[b * SWEEP_BLK + e];
+                        T& x = p[b * SWEEP_BLK + e];
+                        x = k < 0 ? mul_nc(x, y[e]) : x;
+                        k = k < 0 ? SWEEP_ONE : k;
+                    }
+                }
         }
-    };
-    // A slot without a row skips its loads and keeps the (defined) values of an earlier task in
-    // the task and gather registers; nothing computed from them is stored.
-    T g[3][EPL] = {};
-    // X: level lev's task, loaded; Y: level lev + 1's, located; Z receives lev + 2's
-    auto run = [&](SweepTask<T, EPL>& X, SweepTask<T, EPL>& Y, SweepTask<T, EPL>& Z, int lev) {
-        if (X.t >= 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the entries, and this wave's last store
+        auto gather = [&](int b, T(&y)[SWEEP_BLK]) {
 #pragma unroll
-            for (int j = 0; j < EPL; j++)
+            for (int e = 0; e < SWEEP_BLK; e++) y[e] = ring[id[b * SWEEP_BLK + e]];
+        };
+        auto products = [&](int b, const T(&y)[SWEEP_BLK]) {
 #pragma unroll
-                for (int c = 0; c < 3; c++) g[c][j] = v[(size_t)c * N + X.pc[j]];
+            for (int e = 0; e < SWEEP_BLK; e++) p[b * SWEEP_BLK + e] = mul_nc(p[b * SWEEP_BLK + e], y[e]);
+        };
+        auto subtract = [&](int b) {
+#pragma unroll
+            for (int e = 0; e < SWEEP_BLK; e++) s = add_nc(s, -p[b * SWEEP_BLK + e]);
+        };
+        T* const place = ring + ((C.t0 + l) & (SWEEP_RING - 1));
+        // While earlier chunks work, what they have left of this chunk. Forward: block by block from
+        // the first one (first = first block not subtracted), backward: products from the last
+        // block to the first (last = blocks still without), the sum has to wait for block 0.
+        int first = NB - nblk, last = nblk;
+        int d = done();
+        for (;;) {
+            if constexpr (!UPPER) {
+                StaticFor<0, NB>::run([&](auto B) {
+                    constexpr int b = decltype(B)::value;
+                    if (first == b && d >= C.need[b]) {
+                        T y[SWEEP_BLK];
+                        gather(b, y);
+                        products(b, y);
+                        subtract(b);
+                        first = b + 1;
+                    }
+                });
+            } else {
+                StaticFor<0, NB>::run([&](auto B) {
+                    constexpr int b = NB - 1 - decltype(B)::value;
+                    if (last == b + 1 && d >= C.need[b]) {
+                        T y[SWEEP_BLK];
+                        gather(b, y);
+                        products(b, y);
+                        last = b;
+                    }
+                });
+            }
+            if (d >= c - 1) break;
+            if (d < c - 2) __builtin_amdgcn_s_sleep(1);
+            d = done();
         }
-        asm volatile("" ::: "memory");  // the gathers are requested before the later levels' loads
-        load_entries(Y);
-        locate(Z, lev + 2);
-        const int len = X.t >= 0 ? X.e - X.a : 0;
-#pragma unroll
-        for (int j = 0; j < EPL; j++) {
-            const int k = l + j * SL;
-            const bool in = k < len;
-#pragma unroll
-            for (int c = 0; c < 3; c++) P[c][k] = in ? mul_nc(X.pv[j], g[c][j]) : T(0);
+        // next in line: what is left takes one path without branches per number of blocks
+        __builtin_amdgcn_s_setprio(3);
+        while (d != c) d = done();
+        if constexpr (!UPPER) {
+            StaticFor<0, NB>::run([&](auto F) {
+                constexpr int f = decltype(F)::value;
+                if (first == f) {
+                    T y[YB][SWEEP_BLK];  // a block's values are read while the one before is subtracted
+                    gather(f, y[0]);
+                    StaticFor<f, NB>::run([&](auto B) {
+                        constexpr int b = decltype(B)::value;
+                        if constexpr (b + 1 < NB && YB == 2) gather(b + 1, y[(b + 1 - f) % YB]);
+                        products(b, y[(b - f) % YB]);
+                        if constexpr (b + 1 < NB && YB == 1) gather(b + 1, y[0]);
+                        subtract(b);
+                        if constexpr (b + 2 < NB) asm volatile("" ::: "memory");
+                    });
+                    first = NB;
+                }
+            });
+        } else {
+            StaticFor<1, NB + 1>::run([&](auto L) {
+                constexpr int f = decltype(L)::value;
+                if (last == f) {
+                    T y[YB][SWEEP_BLK];
+                    gather(0, y[0]);
+                    StaticFor<0, f>::run([&](auto B) {
+                        constexpr int b = decltype(B)::value;
+                        if constexpr (b + 1 < f && YB == 2) gather(b + 1, y[(b + 1) % YB]);
+                        products(b, y[b % YB]);
+                        if constexpr (b + 1 < f && YB == 1) gather(b + 1, y[0]);
+                        if constexpr (b + 2 < f) asm volatile("" ::: "memory");
+                    });
+                    last = 0;
+                }
+            });
+            StaticFor<0, NB>::run([&](auto B) {
+                if (decltype(B)::value < nblk) subtract(decltype(B)::value);
+            });
+            s = s / dg;
         }
-        wave_sync();
-        // every lane of a slot sums and stores: lanes past 2 repeat lane 2 (same value, same address)
-        T s = X.s;
-#pragma unroll 32
-        for (int k = 0; k < CH; k++) s = add_nc(s, -P[lc][k]);
-        if (UPPER) s = s / X.dg;
-        if (X.t >= 0) v[(size_t)lc * N + X.r] = s;
-        wave_sync();  // the slot's products are read before the next level overwrites them
-        __syncthreads();
-    };
-    SweepTask<T, EPL> A{}, B{}, C{};
-    locate(A, 0);
-    load_entries(A);
-    locate(B, 1);
-    // levels past n_lev are empty (level_start clamps), so the loop body needs no test; the
-    // compiler waits for every outstanding access at the loop head, hence the long body
-    for (int lev = 0; lev < n_lev; lev += 6) {
-        run(A, B, C, lev);
-        run(B, C, A, lev + 1);
-        run(C, A, B, lev + 2);
-        run(A, B, C, lev + 3);
-        run(B, C, A, lev + 4);
-        run(C, A, B, lev + 5);
+        *place = s;  // lanes past the last row write its value again
+        asm volatile("" ::: "memory");  // the values before the count
+        __hip_atomic_store(s_done, c + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __builtin_amdgcn_s_setprio(0);
+        v[r] = s;
     }
 }
 
-// dst[i] = (T) src[map[i]]
+// dst[i] = (T) src[map[i]], 0 where map[i] < 0
 template <typename T>
 __global__ void gather_kernel(const double* __restrict__ src, const int32_t* __restrict__ map, T* __restrict__ dst,
                               int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = (T)src[map[i]];
+    if (i < n) dst[i] = map[i] < 0 ? (T)0 : (T)src[map[i]];
 }
 
 __global__ void to_f32_kernel(const double* __restrict__ in, float* __restrict__ out, size_t n) {
@@ -402,16 +493,21 @@ struct rbfx_stokes {
     // factor of A_L = -eta L in CSR (sorted columns)
     int32_t *ip = nullptr, *col = nullptr, *diag = nullptr;
     double *a_in = nullptr, *f64 = nullptr;
-    int32_t *lrows = nullptr, *loff = nullptr, *urows = nullptr, *uoff = nullptr;
+    int32_t *lrows = nullptr, *loff = nullptr;
     int n_lev_l = 0, n_lev_u = 0;
-    int max_side = 0;  // most entries of a row on one side of the diagonal
-    // the sweeps' packed entries (task order): offsets, columns, source index into the factor,
-    // values in FP64 and FP32, and the diagonal of each backward task
-    int32_t *lpk_off = nullptr, *lpk_col = nullptr, *lpk_src = nullptr;
-    int32_t *upk_off = nullptr, *upk_col = nullptr, *upk_src = nullptr, *upk_dsrc = nullptr;
-    double *lpk64 = nullptr, *upk64 = nullptr, *ud64 = nullptr;
-    float *lpk32 = nullptr, *upk32 = nullptr, *ud32 = nullptr;
-    int l_nnz = 0, u_nnz = 0;
+    // the sweeps: chunks, their tasks' rows, packed entries (places of the values they multiply,
+    // source index into the factor, values in FP64 and FP32), the backward tasks' diagonals
+    struct Side {
+        SweepChunk* chunks = nullptr;
+        int32_t *rows = nullptr, *idx = nullptr, *src64 = nullptr, *src32 = nullptr;
+        double* val64 = nullptr;
+        float* val32 = nullptr;
+        int n_chunks = 0, n_ent = 0;
+    } low, up;
+    int nb = 0;  // the sweeps' variant: blocks of 8 entries a row may take on one side
+    int32_t* udsrc = nullptr;
+    double* ud64 = nullptr;
+    float* ud32 = nullptr;
     // GMRES workspace
     int ws_m = -1;
     void* V = nullptr;    // (m + 1) * n_tot values of the run's type (FP64 size)
@@ -427,11 +523,11 @@ namespace {
 
 void stokes_free(rbfx_stokes* S) {
     for (void* p : {(void*)S->ip, (void*)S->col, (void*)S->diag, (void*)S->a_in, (void*)S->f64,
-                    (void*)S->lrows, (void*)S->loff, (void*)S->urows, (void*)S->uoff, S->V, S->w, (void*)S->r64,
-                    (void*)S->x32d, (void*)S->partial, (void*)S->hbuf, (void*)S->coef, (void*)S->lpk_off,
-                    (void*)S->lpk_col, (void*)S->lpk_src, (void*)S->upk_off, (void*)S->upk_col, (void*)S->upk_src,
-                    (void*)S->upk_dsrc, (void*)S->lpk64, (void*)S->upk64, (void*)S->ud64, (void*)S->lpk32,
-                    (void*)S->upk32, (void*)S->ud32})
+                    (void*)S->lrows, (void*)S->loff, S->V, S->w, (void*)S->r64,
+                    (void*)S->x32d, (void*)S->partial, (void*)S->hbuf, (void*)S->coef, (void*)S->low.chunks,
+                    (void*)S->low.rows, (void*)S->low.idx, (void*)S->low.src64, (void*)S->low.src32, (void*)S->low.val64, (void*)S->low.val32,
+                    (void*)S->up.chunks, (void*)S->up.rows, (void*)S->up.idx, (void*)S->up.src64, (void*)S->up.src32, (void*)S->up.val64,
+                    (void*)S->up.val32, (void*)S->udsrc, (void*)S->ud64, (void*)S->ud32})
         if (p) hipFree(p);
 }
 
@@ -440,6 +536,78 @@ int upload(rbfx_ctx* ctx, T** d, const std::vector<T>& h) {
     if (hipMalloc((void**)d, std::max<size_t>(1, h.size()) * sizeof(T)) != hipSuccess)
         return rbfx_fail(ctx, RBFX_E_NOMEM, "stokes: device allocation of %zu bytes failed", h.size() * sizeof(T));
     if (!h.empty()) RBFX_HIP_CHECK(ctx, hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
+    return RBFX_OK;
+}
+
+struct HostSide {
+    std::vector<SweepChunk> chunks;
+    std::vector<int32_t> rows, idx, src64, src32;
+};
+
+// Chunks and packed entries of one sweep: rows in level order, level l at off[l]; side(r, a, b) gives
+// row r's entries a <= q < b on the sweep's side of the diagonal (columns ascending). Forward, pads
+// come first and block b of nblk is the kernel's block nb - nblk + b (the last entries are the
+// latest solved); backward, pads come last.
+template <typename Fn>
+void pack_side(const std::vector<int32_t>& rows, const std::vector<int32_t>& off, int N, int nb, bool upper, bool fp32,
+               HostSide& D, const Fn& side, const std::vector<int32_t>& col) {
+    D.rows = rows;
+    D.idx.reserve((size_t)N * SWEEP_BLK * 3);
+    D.src64.reserve((size_t)N * SWEEP_BLK * 3);
+    std::vector<int32_t> task(N), chunk(N);  // by row
+    for (int t = 0; t < N; t++) task[rows[t]] = t;
+    for (size_t lev = 0; lev + 1 < off.size(); lev++)
+        for (int t0 = off[lev]; t0 < off[lev + 1]; t0 += SWEEP_ROWS) {
+            SweepChunk C = {};
+            C.t0 = t0;
+            C.nr = std::min(SWEEP_ROWS, off[lev + 1] - t0);
+            C.base = (int)D.idx.size();
+            int most = 0, a, b;
+            for (int l = 0; l < C.nr; l++) {
+                side(rows[t0 + l], a, b);
+                most = std::max(most, b - a);
+                chunk[rows[t0 + l]] = (int)D.chunks.size();
+            }
+            const int nblk = (most + SWEEP_BLK - 1) / SWEEP_BLK, slots = nblk * SWEEP_BLK;
+            D.idx.resize(D.idx.size() + (size_t)slots * C.nr, SWEEP_ZERO);
+            D.src64.resize(D.idx.size(), -1);
+            if (fp32) D.src32.resize(D.idx.size(), -1);
+            int far = 0;
+            for (int l = 0; l < C.nr; l++) {
+                side(rows[t0 + l], a, b);
+                for (int q = a; q < b; q++) {
+                    const int e = upper ? q - a : slots - (b - q);
+                    int& need = C.need[(upper ? 0 : nb - nblk) + e / SWEEP_BLK];
+                    // 16 bytes of a lane side by side: 4 places, 2 or 4 values
+                    auto at = [&](int per) { return (size_t)C.base + (size_t)(e / per * per) * C.nr + per * l + e % per; };
+                    const int k = col[q], tk = task[k];
+                    D.src64[at(2)] = q;
+                    if (fp32) D.src32[at(4)] = q;
+                    if (tk >= t0 - SWEEP_RING) {
+                        D.idx[at(4)] = tk & (SWEEP_RING - 1);
+                        need = std::max(need, chunk[k] + 1);
+                    } else {
+                        D.idx[at(4)] = ~k;
+                        far = 1;
+                    }
+                }
+            }
+            C.nblk = nblk | far << 8;
+            D.chunks.push_back(C);
+        }
+}
+
+int upload_side(rbfx_ctx* ctx, rbfx_stokes::Side& D, const HostSide& H) {
+    D.n_chunks = (int)H.chunks.size();
+    D.n_ent = (int)H.idx.size();
+    int rc;
+    if ((rc = upload(ctx, &D.chunks, H.chunks)) || (rc = upload(ctx, &D.rows, H.rows)) ||
+        (rc = upload(ctx, &D.idx, H.idx)) || (rc = upload(ctx, &D.src64, H.src64)) || (rc = upload(ctx, &D.src32, H.src32)))
+        return rc;
+    const size_t n = std::max<size_t>(1, H.idx.size());
+    if (hipMalloc((void**)&D.val64, n * sizeof(double)) != hipSuccess ||
+        (!H.src32.empty() && hipMalloc((void**)&D.val32, n * sizeof(float)) != hipSuccess))
+        return rbfx_fail(ctx, RBFX_E_NOMEM, "stokes_create: packed factor entries");
     return RBFX_OK;
 }
 
@@ -466,39 +634,35 @@ int apply(rbfx_stokes* S, const T* x, T* y) {
     return RBFX_OK;
 }
 
-template <typename T, bool UPPER>
-void launch_sweep(const rbfx_stokes* S, hipStream_t st, const int32_t* rows, const int32_t* off, int n_lev,
-                  const int32_t* pk_off, const int32_t* pk_col, const T* pk_val, const T* pk_diag, T* v) {
-    const bool lds = n_lev <= SWEEP_LDS_LEVELS;
-    const bool wide = S->max_side > SWEEP_CH;
-    if (lds && !wide)
-        ilu0_sweep_kernel<T, UPPER, true, SWEEP_CH><<<1, SWEEP_THREADS, 0, st>>>(rows, off, n_lev, pk_off, pk_col, pk_val,
-                                                                                pk_diag, S->N, v);
-    else if (lds)
-        ilu0_sweep_kernel<T, UPPER, true, SWEEP_CH_MAX><<<1, SWEEP_THREADS, 0, st>>>(rows, off, n_lev, pk_off, pk_col,
-                                                                                    pk_val, pk_diag, S->N, v);
-    else if (!wide)
-        ilu0_sweep_kernel<T, UPPER, false, SWEEP_CH><<<1, SWEEP_THREADS, 0, st>>>(rows, off, n_lev, pk_off, pk_col,
-                                                                                 pk_val, pk_diag, S->N, v);
-    else
-        ilu0_sweep_kernel<T, UPPER, false, SWEEP_CH_MAX><<<1, SWEEP_THREADS, 0, st>>>(rows, off, n_lev, pk_off, pk_col,
+template <typename T, bool UPPER, int NB>
+void launch_sweep_nb(const rbfx_stokes* S, const rbfx_stokes::Side& D, const T* pk_val, const T* pk_diag, T* v) {
+    const size_t lds = (SWEEP_RING + 2) * sizeof(T) + 16;
+    ilu0_sweep_kernel<T, UPPER, NB><<<3, 64 * sweep_waves(NB), lds, S->ctx->stream>>>(D.chunks, D.n_chunks, D.rows, D.idx,
                                                                                      pk_val, pk_diag, S->N, v);
+}
+
+template <typename T, bool UPPER>
+int launch_sweep(const rbfx_stokes* S, const rbfx_stokes::Side& D, const T* pk_val, const T* pk_diag, T* v) {
+    switch (S->nb) {
+        case 4: launch_sweep_nb<T, UPPER, 4>(S, D, pk_val, pk_diag, v); break;
+        case 5: launch_sweep_nb<T, UPPER, 5>(S, D, pk_val, pk_diag, v); break;
+        case 6: launch_sweep_nb<T, UPPER, 6>(S, D, pk_val, pk_diag, v); break;
+        case 7: launch_sweep_nb<T, UPPER, 7>(S, D, pk_val, pk_diag, v); break;
+        default: launch_sweep_nb<T, UPPER, SWEEP_MAX_BLKS>(S, D, pk_val, pk_diag, v);
+    }
+    RBFX_LAUNCH_CHECK(S->ctx, "ilu0_sweep_kernel");
+    return RBFX_OK;
 }
 
 // v = M^-1 v: both sweeps on the three velocity blocks; the other rows are identity rows.
 template <typename T>
 int precond(rbfx_stokes* S, T* v) {
-    rbfx_ctx* ctx = S->ctx;
-    hipStream_t st = ctx->stream;
     const bool d = sizeof(T) == 8;
-    const T* lv = d ? (const T*)S->lpk64 : (const T*)S->lpk32;
-    const T* uv = d ? (const T*)S->upk64 : (const T*)S->upk32;
+    const T* lv = d ? (const T*)S->low.val64 : (const T*)S->low.val32;
+    const T* uv = d ? (const T*)S->up.val64 : (const T*)S->up.val32;
     const T* ud = d ? (const T*)S->ud64 : (const T*)S->ud32;
-    launch_sweep<T, false>(S, st, S->lrows, S->loff, S->n_lev_l, S->lpk_off, S->lpk_col, lv, nullptr, v);
-    RBFX_LAUNCH_CHECK(ctx, "ilu0_sweep_kernel");
-    launch_sweep<T, true>(S, st, S->urows, S->uoff, S->n_lev_u, S->upk_off, S->upk_col, uv, ud, v);
-    RBFX_LAUNCH_CHECK(ctx, "ilu0_sweep_kernel");
-    return RBFX_OK;
+    const int rc = launch_sweep<T, false>(S, S->low, lv, nullptr, v);
+    return rc ? rc : launch_sweep<T, true>(S, S->up, uv, ud, v);
 }
 
 // out[0..K) = V[0..K)^T w (w == nullptr: plain sums), accumulate: out += instead.
@@ -728,46 +892,23 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     };
     int max_side = 0;
     for (int r = 0; r < N; r++) max_side = std::max({max_side, dg[r] - ip[r], ip[r + 1] - dg[r] - 1});
-    // a sweep runs at most sweep_slots rows per step: larger levels become several steps
-    const int slots = sweep_slots(max_side > SWEEP_CH ? SWEEP_CH_MAX : SWEEP_CH);
-    auto split = [&](std::vector<int32_t>& off) {
-        std::vector<int32_t> o(1, 0);
-        for (size_t l = 0; l + 1 < off.size(); l++) {
-            for (int32_t b = off[l] + slots; b < off[l + 1]; b += slots) o.push_back(b);
-            o.push_back(off[l + 1]);
-        }
-        off.swap(o);
-    };
     std::vector<int32_t> lrows, loff, urows, uoff;
     by_level(lev, nl, lrows, loff);
     by_level(ulev, nu, urows, uoff);
-    split(loff);
-    split(uoff);
-    nl = (int)loff.size() - 1;
-    nu = (int)uoff.size() - 1;
-    // the sweeps' entries packed task by task (level order), columns ascending
-    std::vector<int32_t> lpo(N + 1, 0), lpc, lps, upo(N + 1, 0), upc, ups, uds(N);
-    for (int t = 0; t < N; t++) {
-        const int r = lrows[t];
-        for (int q = ip[r]; q < dg[r]; q++) {
-            lpc.push_back(col[q]);
-            lps.push_back(q);
-        }
-        lpo[t + 1] = (int32_t)lpc.size();
-    }
-    for (int t = 0; t < N; t++) {
-        const int r = urows[t];
-        for (int q = dg[r] + 1; q < ip[r + 1]; q++) {
-            upc.push_back(col[q]);
-            ups.push_back(q);
-        }
-        upo[t + 1] = (int32_t)upc.size();
-        uds[t] = dg[r];
-    }
-    // the sweeps read a whole chunk from any task's start: SWEEP_CH_MAX zero entries past the end
-    const int l_nnz = (int)lpc.size(), u_nnz = (int)upc.size();
-    lpc.resize(l_nnz + SWEEP_CH_MAX, 0);
-    upc.resize(u_nnz + SWEEP_CH_MAX, 0);
+    const int nb = sweep_variant((max_side + SWEEP_BLK - 1) / SWEEP_BLK);
+    HostSide low, up;
+    const bool fp32 = ops32 != nullptr;  // the FP32 copy of the factor serves the FP32 inner solves
+    pack_side(lrows, loff, N, nb, false, fp32, low, [&](int r, int& a, int& b) { a = ip[r], b = dg[r]; }, col);
+    pack_side(urows, uoff, N, nb, true, fp32, up, [&](int r, int& a, int& b) { a = dg[r] + 1, b = ip[r + 1]; }, col);
+    std::vector<int32_t> uds(N);
+    for (int t = 0; t < N; t++) uds[t] = dg[urows[t]];
+    // what rbfx_stokes_info reports: levels in steps of at most 32 rows (16 for wide stencils)
+    const int slots = max_side > 32 ? 16 : 32;
+    auto steps = [&](const std::vector<int32_t>& off) {
+        int n = 0;
+        for (size_t l = 0; l + 1 < off.size(); l++) n += (off[l + 1] - off[l] + slots - 1) / slots;
+        return n;
+    };
 
     rbfx_stokes* S = new rbfx_stokes();
     S->ctx = ctx;
@@ -777,38 +918,24 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     S->N = N;
     S->width = W;
     S->n_tot = 4 * (size_t)N + 4;
-    S->n_lev_l = nl;
-    S->n_lev_u = nu;
-    S->max_side = max_side;
+    S->n_lev_l = steps(loff);
+    S->n_lev_u = steps(uoff);
+    S->nb = nb;
     int rc = RBFX_OK;
     if ((rc = upload(ctx, &S->ip, ip)) || (rc = upload(ctx, &S->col, col)) || (rc = upload(ctx, &S->diag, dg)) ||
         (rc = upload(ctx, &S->a_in, a)) || (rc = upload(ctx, &S->lrows, lrows)) || (rc = upload(ctx, &S->loff, loff)) ||
-        (rc = upload(ctx, &S->urows, urows)) || (rc = upload(ctx, &S->uoff, uoff)) ||
-        (rc = upload(ctx, &S->f64, a)) || (rc = upload(ctx, &S->lpk_off, lpo)) || (rc = upload(ctx, &S->lpk_col, lpc)) ||
-        (rc = upload(ctx, &S->lpk_src, lps)) || (rc = upload(ctx, &S->upk_off, upo)) ||
-        (rc = upload(ctx, &S->upk_col, upc)) || (rc = upload(ctx, &S->upk_src, ups)) ||
-        (rc = upload(ctx, &S->upk_dsrc, uds)) || (rc = workspace(S, 1))) {
+        (rc = upload(ctx, &S->f64, a)) || (rc = upload_side(ctx, S->low, low)) || (rc = upload_side(ctx, S->up, up)) ||
+        (rc = upload(ctx, &S->udsrc, uds)) || (rc = workspace(S, 1))) {
         stokes_free(S);
         delete S;
         return rc;
     }
-    S->l_nnz = l_nnz;
-    S->u_nnz = u_nnz;
-    const size_t ln = lpc.size(), un = upc.size();  // with the zero entries past the end
-    if (hipMalloc((void**)&S->lpk64, ln * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&S->upk64, un * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&S->ud64, N * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&S->lpk32, ln * sizeof(float)) != hipSuccess ||
-        hipMalloc((void**)&S->upk32, un * sizeof(float)) != hipSuccess ||
-        hipMalloc((void**)&S->ud32, N * sizeof(float)) != hipSuccess) {
+    if (hipMalloc((void**)&S->ud64, N * sizeof(double)) != hipSuccess || hipMalloc((void**)&S->ud32, N * sizeof(float)) != hipSuccess) {
         stokes_free(S);
         delete S;
         return rbfx_fail(ctx, RBFX_E_NOMEM, "stokes_create: packed factor entries");
     }
-    hipError_t e = hipMemsetAsync(S->lpk64, 0, ln * sizeof(double), ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(S->upk64, 0, un * sizeof(double), ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(S->lpk32, 0, ln * sizeof(float), ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(S->upk32, 0, un * sizeof(float), ctx->stream);
+    hipError_t e = hipSuccess;
     if (e == hipSuccess) {
         ilu0_factor_kernel<<<1, FACTOR_THREADS, 0, ctx->stream>>>(S->ip, S->col, S->diag, S->a_in, S->lrows, S->loff, nl,
                                                                   N * W, S->f64);
@@ -816,16 +943,14 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     }
     if (e == hipSuccess) {
         hipStream_t st = ctx->stream;
-        if (S->l_nnz) {
-            gather_kernel<double><<<blocks_for(S->l_nnz, 256), 256, 0, st>>>(S->f64, S->lpk_src, S->lpk64, S->l_nnz);
-            gather_kernel<float><<<blocks_for(S->l_nnz, 256), 256, 0, st>>>(S->f64, S->lpk_src, S->lpk32, S->l_nnz);
+        for (rbfx_stokes::Side* D : {&S->low, &S->up}) {
+            if (!D->n_ent) continue;
+            gather_kernel<double><<<blocks_for(D->n_ent, 256), 256, 0, st>>>(S->f64, D->src64, D->val64, D->n_ent);
+            if (D->val32)
+                gather_kernel<float><<<blocks_for(D->n_ent, 256), 256, 0, st>>>(S->f64, D->src32, D->val32, D->n_ent);
         }
-        if (S->u_nnz) {
-            gather_kernel<double><<<blocks_for(S->u_nnz, 256), 256, 0, st>>>(S->f64, S->upk_src, S->upk64, S->u_nnz);
-            gather_kernel<float><<<blocks_for(S->u_nnz, 256), 256, 0, st>>>(S->f64, S->upk_src, S->upk32, S->u_nnz);
-        }
-        gather_kernel<double><<<blocks_for(N, 256), 256, 0, st>>>(S->f64, S->upk_dsrc, S->ud64, N);
-        gather_kernel<float><<<blocks_for(N, 256), 256, 0, st>>>(S->f64, S->upk_dsrc, S->ud32, N);
+        gather_kernel<double><<<blocks_for(N, 256), 256, 0, st>>>(S->f64, S->udsrc, S->ud64, N);
+        gather_kernel<float><<<blocks_for(N, 256), 256, 0, st>>>(S->f64, S->udsrc, S->ud32, N);
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
