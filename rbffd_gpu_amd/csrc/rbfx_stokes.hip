@@ -18,9 +18,9 @@
 // component), with identity rows elsewhere. The factor of -eta L is computed once and applied
 // to the three components. The dependencies of the factorization and of both sweeps follow
 // the stencil graph; rows are grouped into dependency levels on the host (a row's level is one
-// more than the deepest of the rows it reads). The factorization runs them on one workgroup with a
-// barrier between levels; each sweep runs the three components on a workgroup each, its waves
-// handing the levels on through a counter in LDS. Every row accumulates in the reference's
+// more than the deepest of the rows it reads). The factorization runs a wave per row on the whole
+// device, each entry its own signal; each sweep runs the three components on a workgroup each, its
+// waves handing the levels on through a counter in LDS. Every row accumulates in the reference's
 // order, without fused multiply-adds, so the factor and the sweeps match the CPU restatement bit
 // for bit.
 //
@@ -28,6 +28,7 @@
 // the basis and one multi-axpy), Givens rotations on the host. The stopping test is the
 // reference's: the estimate of ||M^-1 (b - A x)|| / ||b|| below tol.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -36,8 +37,11 @@
 
 namespace {
 
-constexpr int FACTOR_THREADS = 1024;
-constexpr int FACTOR_WAVES = FACTOR_THREADS / 64;
+constexpr int FACTOR_WAVES = 4;       // per workgroup
+constexpr int FACTOR_BLOCKS = 256;
+constexpr int FACTOR_AHEAD = 2;       // lower entries whose values a wave asks for at once
+// What a factor entry holds until it is computed: a signalling NaN, which no operation returns.
+constexpr unsigned long long FACTOR_UNSET = 0x7ff4a5a5a5a5a5a5ull;
 // A sweep's variants hold rows of up to 32, 40, 48 or 64 entries on one side of the diagonal in
 // registers: 12 waves of at most 168 VGPRs for the first, 8 of at most 256 for the others.
 constexpr int sweep_variant(int blks) { return blks <= 4 ? 4 : blks <= 7 ? blks : 8; }
@@ -48,7 +52,6 @@ constexpr int SWEEP_MAX_BLKS = 8;  // up to 64 entries of a row on one side of t
 constexpr int SWEEP_RING = 16384;  // solved values kept in LDS: the last 16384 tasks
 constexpr int SWEEP_ZERO = SWEEP_RING, SWEEP_ONE = SWEEP_RING + 1;  // LDS places holding 0 and 1
 constexpr int FACTOR_MAX_WIDTH = 64;  // one lane per stencil entry in the factorization
-constexpr int FACTOR_CHUNK = 8;       // L entries whose U rows a wave loads at once
 constexpr int DOT_THREADS = 256;
 constexpr int DOT_BLOCKS = 256;
 
@@ -171,85 +174,119 @@ __global__ void constraint_rows_kernel(const double* __restrict__ sums, int N, T
     if (threadIdx.x < 4) y[4 * (size_t)N + threadIdx.x] = (T)sums[threadIdx.x];
 }
 
-// ILU(0) of A_L (CSR, sorted columns, diagonal present) in dependency levels. One wave per row:
-// lane q holds entry q of the row in LDS; for every L entry k (ascending) the multiplier
-// t = w_k / U_kk is formed and the lanes that hold row k's U entries subtract t * U_kj from the
-// row's entry j where the input holds a nonzero (no fill). Nothing but w depends on the order of
-// the L entries, so for FACTOR_CHUNK of them at a time the wave first loads, all at once, each
-// row k's U entries and finds where their columns sit in the row (or that they do not, or that
-// the input holds a zero there); the ordered part then only reads LDS.
-__global__ void __launch_bounds__(FACTOR_THREADS) ilu0_factor_kernel(const int32_t* __restrict__ ip,
-                                                                    const int32_t* __restrict__ col,
-                                                                    const int32_t* __restrict__ diag,
-                                                                    const double* __restrict__ a_in,
-                                                                    const int32_t* __restrict__ rows,
-                                                                    const int32_t* __restrict__ off, int n_lev,
-                                                                    int nnz, double* __restrict__ f) {
-    __shared__ double wv[FACTOR_WAVES][FACTOR_MAX_WIDTH];
-    __shared__ int wc[FACTOR_WAVES][FACTOR_MAX_WIDTH];
-    __shared__ double ukk[FACTOR_WAVES][FACTOR_MAX_WIDTH];
-    __shared__ int upos[FACTOR_WAVES][FACTOR_CHUNK][FACTOR_MAX_WIDTH];  // position in the row, -1: none
-    __shared__ double uval[FACTOR_WAVES][FACTOR_CHUNK][FACTOR_MAX_WIDTH];
-    const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    for (int lev = 0; lev < n_lev; lev++) {
-        const int r0 = off[lev], r1 = off[lev + 1];
-        for (int ri = r0 + wave; ri < r1; ri += FACTOR_WAVES) {
-            const int r = rows[ri];
-            const int s = ip[r], len = ip[r + 1] - s, dpos = diag[r] - s;
-            bool nz = false;
-            if (lane < len) {
-                wv[wave][lane] = a_in[s + lane];
-                wc[wave][lane] = col[s + lane];
-                nz = a_in[s + lane] != 0.0;
+// ILU(0) of A_L (N rows of W entries, columns ascending, diagonal at diag[r]), one wave per row, lane
+// p holding entry p. For every lower entry q (ascending, column k): t = w_q / U_kk, and every later
+// entry whose column row k's upper part holds, if the input is not zero there, subtracts t * U_kj.
+// Each entry sees its updates in that order, without fused multiply-adds, as the reference.
+//
+// Rows are taken from a counter in level order, and a row's values are their own signal: f starts
+// at FACTOR_UNSET everywhere, a row's entries are stored as single 8-byte values in device scope, and a
+// wave asks for the entries it needs (up to FACTOR_AHEAD rows k at once) until they are set. Where row k's
+// columns sit in the row does not depend on values and is found while earlier rows are computed:
+// upos[q][p] is the upper entry of row k = column q that updates entry p.
+// Every wait ends: a row's entries come from rows of lower levels, which were taken from the counter
+// before it and run in waves that are resident; the lowest unfinished row waits for nothing.
+//
+// Bound: latency, per level one value from another CU and then a division and an update per lower
+// entry left. N = 40962, n = 31 (1735 levels): 1.6 ms, 0.9 us per level; one workgroup of 16 waves
+// with a barrier per level took 56.7 ms. Asking for 1, 4 and 8 rows at once: 1.6, 2.1 and 2.9 ms;
+// 128 and 512 workgroups: 1.8 and 1.7 ms.
+__global__ void __launch_bounds__(64 * FACTOR_WAVES) ilu0_factor_kernel(const int32_t* __restrict__ col,
+                                                                       const int32_t* __restrict__ diag,
+                                                                       const double* __restrict__ a_in,
+                                                                       const int32_t* __restrict__ rows, int N, int W,
+                                                                       int* counter, double* f) {
+    __shared__ int s_col[FACTOR_WAVES][FACTOR_MAX_WIDTH];
+    __shared__ uint8_t s_upos[FACTOR_WAVES][FACTOR_MAX_WIDTH][FACTOR_MAX_WIDTH];
+    constexpr int NONE = 255;
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    int(&wc)[FACTOR_MAX_WIDTH] = s_col[wave];
+    uint8_t(&upos)[FACTOR_MAX_WIDTH][FACTOR_MAX_WIDTH] = s_upos[wave];
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto value = [&](int q) {
+        return __hip_atomic_load((unsigned long long*)f + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    for (;;) {
+        int t = 0;
+        if (lane == 0) t = atomicAdd(counter, 1);
+        t = __builtin_amdgcn_readfirstlane(t);
+        if (t >= N) return;
+        const int r = rows[t];
+        const bool in = lane < W;
+        const int c = in ? col[r * W + lane] : INT_MAX;
+        double w = in ? a_in[r * W + lane] : 0.0;
+        const bool nz = w != 0.0;  // entries the input holds: updates allowed
+        const int dpos = diag[r] - r * W;
+        const int dk = lane < dpos ? diag[c] : 0;  // lane q: place of the diagonal of row k = column q
+        wave_sync();                               // the last row's places have been read
+        wc[lane] = c;
+        for (int q = 0; q < dpos; q++) upos[q][lane] = NONE;
+        wave_sync();
+        for (int q0 = 0; q0 < dpos; q0 += 8) {
+            int j[8];
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                const int q = q0 + b < dpos ? q0 + b : q0;
+                const int d = __builtin_amdgcn_readlane(dk, q), k = __builtin_amdgcn_readlane(c, q);
+                const int at = d + 1 + lane;
+                j[b] = at < (k + 1) * W ? col[at] : INT_MAX;
             }
-            const uint64_t nzmask = __ballot(nz);  // entries the input holds (updates allowed)
-            __builtin_amdgcn_wave_barrier();
-            for (int q0 = 0; q0 < dpos; q0 += FACTOR_CHUNK) {
-                const int nq = dpos - q0 < FACTOR_CHUNK ? dpos - q0 : FACTOR_CHUNK;
-                if (lane < nq) ukk[wave][lane] = f[diag[wc[wave][q0 + lane]]];
-                // all loads of the chunk first (addresses clamped into the arrays), then the searches
-                int ud[FACTOR_CHUNK], ue[FACTOR_CHUNK], uj[FACTOR_CHUNK];
-                double uu[FACTOR_CHUNK];
 #pragma unroll
-                for (int c = 0; c < FACTOR_CHUNK; c++) ud[c] = diag[wc[wave][q0 + (c < nq ? c : 0)]];
-#pragma unroll
-                for (int c = 0; c < FACTOR_CHUNK; c++) {
-                    const int q = ud[c] + 1 + lane < nnz ? ud[c] + 1 + lane : nnz - 1;
-                    ue[c] = ip[wc[wave][q0 + (c < nq ? c : 0)] + 1];
-                    uj[c] = col[q];
-                    uu[c] = f[q];
+            for (int b = 0; b < 8; b++) {
+                int lo = 0, hi = W;  // j[b] among the row's ascending columns
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (wc[mid] < j[b]) lo = mid + 1; else hi = mid;
                 }
-#pragma unroll
-                for (int c = 0; c < FACTOR_CHUNK; c++) {
-                    int pos = -1;
-                    if (c < nq && lane < ue[c] - ud[c] - 1) {
-                        const int j = uj[c];
-                        int lo = 0, hi = len;  // find j among the row's sorted columns
-                        while (lo < hi) {
-                            const int mid = (lo + hi) >> 1;
-                            if (wc[wave][mid] < j) lo = mid + 1; else hi = mid;
-                        }
-                        if (lo < len && wc[wave][lo] == j && ((nzmask >> lo) & 1)) pos = lo;
-                    }
-                    upos[wave][c][lane] = pos;
-                    uval[wave][c][lane] = uu[c];
-                }
-                __builtin_amdgcn_wave_barrier();
-                for (int c = 0; c < nq; c++) {
-                    const int qq = q0 + c;
-                    const double t = wv[wave][qq] / ukk[wave][c];
-                    __builtin_amdgcn_wave_barrier();
-                    if (lane == 0) wv[wave][qq] = t;
-                    const int pos = upos[wave][c][lane];
-                    if (pos >= 0) wv[wave][pos] = dadd_nc(wv[wave][pos], -dmul_nc(t, uval[wave][c][lane]));
-                    __builtin_amdgcn_wave_barrier();
-                }
+                if (q0 + b < dpos && lo < W && wc[lo] == j[b]) upos[q0 + b][lo] = (uint8_t)lane;
             }
-            if (lane < len) f[s + lane] = wv[wave][lane];
-            __builtin_amdgcn_wave_barrier();
         }
-        __syncthreads();
+        wave_sync();
+        for (int q = 0; q < dpos;) {
+            int u[FACTOR_AHEAD];
+            unsigned long long x[FACTOR_AHEAD], d[FACTOR_AHEAD];
+#pragma unroll
+            for (int b = 0; b < FACTOR_AHEAD; b++) {
+                const int qq = q + b < dpos ? q + b : q;
+                const int at = __builtin_amdgcn_readlane(dk, qq);
+                u[b] = nz ? upos[qq][lane] : NONE;
+                d[b] = value(at);
+                x[b] = u[b] != NONE ? value(at + 1 + u[b]) : 0;
+            }
+            bool go = true;
+            int n = 0;
+#pragma unroll
+            for (int b = 0; b < FACTOR_AHEAD; b++)
+                if (go && q + b < dpos) {
+                    go = !__any(d[b] == FACTOR_UNSET || x[b] == FACTOR_UNSET);
+                    if (go) {
+                        const unsigned long long wb = (unsigned long long)__double_as_longlong(w);
+                        const int lo = __builtin_amdgcn_readlane((int)wb, q + b);
+                        const int hi = __builtin_amdgcn_readlane((int)(wb >> 32), q + b);
+                        const double wq = __longlong_as_double((long long)((unsigned long long)(unsigned)hi << 32 | (unsigned)lo));
+                        const double m = wq / __longlong_as_double((long long)d[b]);
+                        if (u[b] != NONE) w = dadd_nc(w, -dmul_nc(m, __longlong_as_double((long long)x[b])));
+                        if (lane == q + b) w = m;
+                        n++;
+                    }
+                }
+            q += n;
+            if (n == 0) __builtin_amdgcn_s_sleep(1);
+        }
+        unsigned long long out = (unsigned long long)__double_as_longlong(w);
+        if (out == FACTOR_UNSET) out |= 1ull << 51;  // an input NaN of that value, made quiet
+        if (in) __hip_atomic_store((unsigned long long*)f + r * W + lane, out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+__global__ void factor_init_kernel(unsigned long long* f, size_t n, int* counter) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) f[i] = FACTOR_UNSET;
+    if (i == 0) *counter = 0;
 }
 
 // One triangular sweep of the factor over one velocity block (blockIdx.x: u, v or w; the three do
@@ -491,9 +528,9 @@ struct rbfx_stokes {
     int N = 0, width = 0;
     size_t n_tot = 0;
     // factor of A_L = -eta L in CSR (sorted columns)
-    int32_t *ip = nullptr, *col = nullptr, *diag = nullptr;
+    int32_t *col = nullptr, *diag = nullptr;
+    int* counter = nullptr;  // the factorization's next row
     double *a_in = nullptr, *f64 = nullptr;
-    int32_t *lrows = nullptr, *loff = nullptr;
     int n_lev_l = 0, n_lev_u = 0;
     // the sweeps: chunks, their tasks' rows, packed entries (places of the values they multiply,
     // source index into the factor, values in FP64 and FP32), the backward tasks' diagonals
@@ -522,8 +559,7 @@ struct rbfx_stokes {
 namespace {
 
 void stokes_free(rbfx_stokes* S) {
-    for (void* p : {(void*)S->ip, (void*)S->col, (void*)S->diag, (void*)S->a_in, (void*)S->f64,
-                    (void*)S->lrows, (void*)S->loff, S->V, S->w, (void*)S->r64,
+    for (void* p : {(void*)S->col, (void*)S->diag, (void*)S->counter, (void*)S->a_in, (void*)S->f64, S->V, S->w, (void*)S->r64,
                     (void*)S->x32d, (void*)S->partial, (void*)S->hbuf, (void*)S->coef, (void*)S->low.chunks,
                     (void*)S->low.rows, (void*)S->low.idx, (void*)S->low.src64, (void*)S->low.src32, (void*)S->low.val64, (void*)S->low.val32,
                     (void*)S->up.chunks, (void*)S->up.rows, (void*)S->up.idx, (void*)S->up.src64, (void*)S->up.src32, (void*)S->up.val64,
@@ -922,23 +958,26 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     S->n_lev_u = steps(uoff);
     S->nb = nb;
     int rc = RBFX_OK;
-    if ((rc = upload(ctx, &S->ip, ip)) || (rc = upload(ctx, &S->col, col)) || (rc = upload(ctx, &S->diag, dg)) ||
-        (rc = upload(ctx, &S->a_in, a)) || (rc = upload(ctx, &S->lrows, lrows)) || (rc = upload(ctx, &S->loff, loff)) ||
-        (rc = upload(ctx, &S->f64, a)) || (rc = upload_side(ctx, S->low, low)) || (rc = upload_side(ctx, S->up, up)) ||
+    if ((rc = upload(ctx, &S->col, col)) || (rc = upload(ctx, &S->diag, dg)) || (rc = upload(ctx, &S->a_in, a)) ||
+        (rc = upload_side(ctx, S->low, low)) || (rc = upload_side(ctx, S->up, up)) ||
         (rc = upload(ctx, &S->udsrc, uds)) || (rc = workspace(S, 1))) {
         stokes_free(S);
         delete S;
         return rc;
     }
-    if (hipMalloc((void**)&S->ud64, N * sizeof(double)) != hipSuccess || hipMalloc((void**)&S->ud32, N * sizeof(float)) != hipSuccess) {
+    if (hipMalloc((void**)&S->f64, (size_t)N * W * sizeof(double)) != hipSuccess ||
+        hipMalloc((void**)&S->counter, sizeof(int)) != hipSuccess ||
+        hipMalloc((void**)&S->ud64, N * sizeof(double)) != hipSuccess || hipMalloc((void**)&S->ud32, N * sizeof(float)) != hipSuccess) {
         stokes_free(S);
         delete S;
         return rbfx_fail(ctx, RBFX_E_NOMEM, "stokes_create: packed factor entries");
     }
     hipError_t e = hipSuccess;
     if (e == hipSuccess) {
-        ilu0_factor_kernel<<<1, FACTOR_THREADS, 0, ctx->stream>>>(S->ip, S->col, S->diag, S->a_in, S->lrows, S->loff, nl,
-                                                                  N * W, S->f64);
+        const size_t nnz = (size_t)N * W;
+        factor_init_kernel<<<blocks_for(nnz, 256), 256, 0, ctx->stream>>>((unsigned long long*)S->f64, nnz, S->counter);
+        ilu0_factor_kernel<<<FACTOR_BLOCKS, 64 * FACTOR_WAVES, 0, ctx->stream>>>(S->col, S->diag, S->a_in, S->low.rows, N, W,
+                                                                                S->counter, S->f64);
         e = hipGetLastError();
     }
     if (e == hipSuccess) {
