@@ -283,10 +283,13 @@ __global__ void __launch_bounds__(64 * FACTOR_WAVES) ilu0_factor_kernel(const in
     }
 }
 
-__global__ void factor_init_kernel(unsigned long long* f, size_t n, int* counter) {
+__global__ void factor_init_kernel(unsigned long long* f, size_t n, int* counter, int* err) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) f[i] = FACTOR_UNSET;
-    if (i == 0) *counter = 0;
+    if (i == 0) {
+        *counter = 0;
+        *err = INT_MAX;
+    }
 }
 
 // One triangular sweep of the factor over one velocity block (blockIdx.x: u, v or w; the three do
@@ -503,12 +506,90 @@ __global__ void __launch_bounds__(64 * sweep_waves(NB)) ilu0_sweep_kernel(const 
     }
 }
 
-// dst[i] = (T) src[map[i]], 0 where map[i] < 0
-template <typename T>
-__global__ void gather_kernel(const double* __restrict__ src, const int32_t* __restrict__ map, T* __restrict__ dst,
-                              int n) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) dst[i] = map[i] < 0 ? (T)0 : (T)src[map[i]];
+// A_L = -eta L by rows with each row's columns ascending (the reference's compressed_matrix), and
+// the places of the diagonals, one wave per layout position; the stencils come from the operator
+// set's layout, L is its first operator. err receives the first position whose stencil holds a
+// node twice or misses its centre.
+__global__ void __launch_bounds__(256) stokes_rows_kernel(const int32_t* __restrict__ idx_t, const double* __restrict__ w_t,
+                                                         const int32_t* __restrict__ order, int N, int W, double eta,
+                                                         int32_t* __restrict__ col, double* __restrict__ a,
+                                                         int32_t* __restrict__ diag, int* __restrict__ err) {
+    const int p = blockIdx.x * 4 + (int)threadIdx.x / 64, lane = threadIdx.x % 64;
+    if (p >= N) return;  // uniform over the wave
+    const int r = ell_row_at(order, p);
+    const size_t e = ell_row_base(p, W) + (size_t)(lane < W ? lane : 0) * ELL_TILE;
+    const int c = lane < W ? idx_t[e] : INT_MAX;
+    const double v = lane < W ? w_t[e * 4] : 0.0;
+    int place = 0;
+    bool twice = false;
+    for (int q = 0; q < W; q++) {
+        const int o = __builtin_amdgcn_readlane(c, q);
+        place += o < c;
+        twice |= o == c && q != lane;
+    }
+    const bool bad = __any(lane < W && twice) || !__any(lane < W && c == r);
+    if (bad) {
+        if (lane == 0) atomicMin(err, p);
+        return;
+    }
+    if (lane < W) {
+        col[(size_t)r * W + place] = c;
+        a[(size_t)r * W + place] = dmul_nc(-eta, v);
+        if (c == r) diag[r] = r * W + place;
+    }
+}
+
+// Packs one sweep's entries from the factor f, one wave per chunk (t0, nr, base and nblk given):
+// where their values lie, the entries in FP64 and (val32 given) FP32, which chunks each block of 8
+// waits for, and the rows' diagonals (dg64 given). Forward, pads come first and block b of nblk is
+// the sweep's block nb - nblk + b (the last entries are the latest solved); backward, pads come last.
+// 16 bytes of a lane lie side by side: 4 places, 2 or 4 values.
+__global__ void __launch_bounds__(256) pack_sweep_kernel(SweepChunk* __restrict__ chunks, int n_chunks,
+                                                        const int32_t* __restrict__ rows, const int32_t* __restrict__ task,
+                                                        const int32_t* __restrict__ chunk_of, const int32_t* __restrict__ col,
+                                                        const int32_t* __restrict__ diag, const double* __restrict__ f, int W,
+                                                        int nb, int upper, int32_t* __restrict__ idx,
+                                                        double* __restrict__ val64, float* __restrict__ val32,
+                                                        double* __restrict__ dg64, float* __restrict__ dg32) {
+    const int c = blockIdx.x * 4 + (int)threadIdx.x / 64, lane = threadIdx.x % 64;
+    if (c >= n_chunks) return;  // uniform over the wave
+    const int t0 = chunks[c].t0, nr = chunks[c].nr, base = chunks[c].base, nblk = chunks[c].nblk;
+    const bool in = lane < nr;
+    const int r = rows[t0 + (in ? lane : 0)], dr = diag[r];
+    const int a = upper ? dr + 1 : r * W, b = upper ? (r + 1) * W : dr;
+    bool far = false;
+    for (int blk = 0; blk < nblk; blk++) {
+        int need = 0;
+        for (int e = blk * SWEEP_BLK; e < (blk + 1) * SWEEP_BLK; e++) {
+            const int q = upper ? a + e : b - (nblk * SWEEP_BLK - e);
+            int at = SWEEP_ZERO;
+            double v = 0.0;
+            if (in && q >= a && q < b) {
+                const int k = col[q], tk = task[k];
+                v = f[q];
+                if (tk >= t0 - SWEEP_RING) {
+                    at = tk & (SWEEP_RING - 1);
+                    need = max(need, chunk_of[k] + 1);
+                } else {
+                    at = ~k;
+                    far = true;
+                }
+            }
+            if (in) {
+                const size_t at4 = (size_t)base + (size_t)(e / 4 * 4) * nr + 4 * lane + e % 4;
+                idx[at4] = at;
+                val64[(size_t)base + (size_t)(e / 2 * 2) * nr + 2 * lane + e % 2] = v;
+                if (val32) val32[at4] = (float)v;
+            }
+        }
+        for (int o = 32; o > 0; o >>= 1) need = max(need, __shfl_xor(need, o));
+        if (lane == 0) chunks[c].need[(upper ? 0 : nb - nblk) + blk] = need;
+    }
+    if (__any(far) && lane == 0) chunks[c].nblk = nblk | 256;
+    if (dg64 && in) {
+        dg64[t0 + lane] = f[dr];
+        if (dg32) dg32[t0 + lane] = (float)f[dr];
+    }
 }
 
 __global__ void to_f32_kernel(const double* __restrict__ in, float* __restrict__ out, size_t n) {
@@ -527,22 +608,23 @@ struct rbfx_stokes {
     double eta = 1.0;
     int N = 0, width = 0;
     size_t n_tot = 0;
-    // factor of A_L = -eta L in CSR (sorted columns)
+    void* rows_mem = nullptr;   // one allocation: col, diag, a_in, f64, counter, err, low.rows
+    void* sweep_mem = nullptr;  // one allocation: the sweeps' arrays
+    // A_L = -eta L and its factor, N rows of the stencil width, columns ascending
     int32_t *col = nullptr, *diag = nullptr;
-    int* counter = nullptr;  // the factorization's next row
     double *a_in = nullptr, *f64 = nullptr;
+    int *counter = nullptr, *err = nullptr;  // the factorization's next row; first bad stencil
     int n_lev_l = 0, n_lev_u = 0;
     // the sweeps: chunks, their tasks' rows, packed entries (places of the values they multiply,
-    // source index into the factor, values in FP64 and FP32), the backward tasks' diagonals
+    // values in FP64 and FP32), the backward tasks' diagonals
     struct Side {
         SweepChunk* chunks = nullptr;
-        int32_t *rows = nullptr, *idx = nullptr, *src64 = nullptr, *src32 = nullptr;
+        int32_t *rows = nullptr, *task = nullptr, *chunk_of = nullptr, *idx = nullptr;
         double* val64 = nullptr;
         float* val32 = nullptr;
-        int n_chunks = 0, n_ent = 0;
+        int n_chunks = 0;
     } low, up;
     int nb = 0;  // the sweeps' variant: blocks of 8 entries a row may take on one side
-    int32_t* udsrc = nullptr;
     double* ud64 = nullptr;
     float* ud32 = nullptr;
     // GMRES workspace
@@ -559,92 +641,78 @@ struct rbfx_stokes {
 namespace {
 
 void stokes_free(rbfx_stokes* S) {
-    for (void* p : {(void*)S->col, (void*)S->diag, (void*)S->counter, (void*)S->a_in, (void*)S->f64, S->V, S->w, (void*)S->r64,
-                    (void*)S->x32d, (void*)S->partial, (void*)S->hbuf, (void*)S->coef, (void*)S->low.chunks,
-                    (void*)S->low.rows, (void*)S->low.idx, (void*)S->low.src64, (void*)S->low.src32, (void*)S->low.val64, (void*)S->low.val32,
-                    (void*)S->up.chunks, (void*)S->up.rows, (void*)S->up.idx, (void*)S->up.src64, (void*)S->up.src32, (void*)S->up.val64,
-                    (void*)S->up.val32, (void*)S->udsrc, (void*)S->ud64, (void*)S->ud32})
+    for (void* p : {S->rows_mem, S->sweep_mem, S->V, S->w, (void*)S->r64, (void*)S->x32d, (void*)S->partial,
+                    (void*)S->hbuf, (void*)S->coef})
         if (p) hipFree(p);
 }
 
-template <typename T>
-int upload(rbfx_ctx* ctx, T** d, const std::vector<T>& h) {
-    if (hipMalloc((void**)d, std::max<size_t>(1, h.size()) * sizeof(T)) != hipSuccess)
-        return rbfx_fail(ctx, RBFX_E_NOMEM, "stokes: device allocation of %zu bytes failed", h.size() * sizeof(T));
-    if (!h.empty()) RBFX_HIP_CHECK(ctx, hipMemcpy(*d, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice));
-    return RBFX_OK;
-}
-
-struct HostSide {
-    std::vector<SweepChunk> chunks;
-    std::vector<int32_t> rows, idx, src64, src32;
+// Pieces of one allocation, each on 256 bytes: carve once without memory for the size, then with it.
+struct Carver {
+    unsigned char* base = nullptr;
+    size_t used = 0;
+    template <typename T>
+    void take(T** p, size_t n) {
+        if (base) *p = reinterpret_cast<T*>(base + used);
+        used += (n * sizeof(T) + 255) / 256 * 256;
+    }
 };
 
-// Chunks and packed entries of one sweep: rows in level order, level l at off[l]; side(r, a, b) gives
-// row r's entries a <= q < b on the sweep's side of the diagonal (columns ascending). Forward, pads
-// come first and block b of nblk is the kernel's block nb - nblk + b (the last entries are the
-// latest solved); backward, pads come last.
+// One sweep's order on the host: rows level by level, each row's task and chunk, and the chunks
+// (up to SWEEP_ROWS rows of a level) with the place of their packed entries.
+struct HostSide {
+    std::vector<SweepChunk> chunks;
+    std::vector<int32_t> rows, task, chunk_of, off;
+    size_t n_ent = 0;
+};
+
+// lev[r] of n_lev levels; count(r): entries of row r on the sweep's side of the diagonal.
 template <typename Fn>
-void pack_side(const std::vector<int32_t>& rows, const std::vector<int32_t>& off, int N, int nb, bool upper, bool fp32,
-               HostSide& D, const Fn& side, const std::vector<int32_t>& col) {
-    D.rows = rows;
-    D.idx.reserve((size_t)N * SWEEP_BLK * 3);
-    D.src64.reserve((size_t)N * SWEEP_BLK * 3);
-    std::vector<int32_t> task(N), chunk(N);  // by row
-    for (int t = 0; t < N; t++) task[rows[t]] = t;
-    for (size_t lev = 0; lev + 1 < off.size(); lev++)
-        for (int t0 = off[lev]; t0 < off[lev + 1]; t0 += SWEEP_ROWS) {
+void order_side(const std::vector<int32_t>& lev, int n_lev, const Fn& count, HostSide& D) {
+    const int N = (int)lev.size();
+    D.off.assign(n_lev + 1, 0);
+    for (int r = 0; r < N; r++) D.off[lev[r] + 1]++;
+    for (int l = 0; l < n_lev; l++) D.off[l + 1] += D.off[l];
+    D.rows.resize(N);
+    D.task.resize(N);
+    D.chunk_of.resize(N);
+    std::vector<int32_t> pos(D.off.begin(), D.off.end() - 1);
+    for (int r = 0; r < N; r++) {
+        const int t = pos[lev[r]]++;
+        D.rows[t] = r;
+        D.task[r] = t;
+    }
+    for (int l = 0; l < n_lev; l++)
+        for (int t0 = D.off[l]; t0 < D.off[l + 1]; t0 += SWEEP_ROWS) {
             SweepChunk C = {};
             C.t0 = t0;
-            C.nr = std::min(SWEEP_ROWS, off[lev + 1] - t0);
-            C.base = (int)D.idx.size();
-            int most = 0, a, b;
-            for (int l = 0; l < C.nr; l++) {
-                side(rows[t0 + l], a, b);
-                most = std::max(most, b - a);
-                chunk[rows[t0 + l]] = (int)D.chunks.size();
+            C.nr = std::min(SWEEP_ROWS, D.off[l + 1] - t0);
+            C.base = (int)D.n_ent;
+            int most = 0;
+            for (int t = t0; t < t0 + C.nr; t++) {
+                const int r = D.rows[t];
+                most = std::max(most, count(r));
+                D.chunk_of[r] = (int)D.chunks.size();
             }
-            const int nblk = (most + SWEEP_BLK - 1) / SWEEP_BLK, slots = nblk * SWEEP_BLK;
-            D.idx.resize(D.idx.size() + (size_t)slots * C.nr, SWEEP_ZERO);
-            D.src64.resize(D.idx.size(), -1);
-            if (fp32) D.src32.resize(D.idx.size(), -1);
-            int far = 0;
-            for (int l = 0; l < C.nr; l++) {
-                side(rows[t0 + l], a, b);
-                for (int q = a; q < b; q++) {
-                    const int e = upper ? q - a : slots - (b - q);
-                    int& need = C.need[(upper ? 0 : nb - nblk) + e / SWEEP_BLK];
-                    // 16 bytes of a lane side by side: 4 places, 2 or 4 values
-                    auto at = [&](int per) { return (size_t)C.base + (size_t)(e / per * per) * C.nr + per * l + e % per; };
-                    const int k = col[q], tk = task[k];
-                    D.src64[at(2)] = q;
-                    if (fp32) D.src32[at(4)] = q;
-                    if (tk >= t0 - SWEEP_RING) {
-                        D.idx[at(4)] = tk & (SWEEP_RING - 1);
-                        need = std::max(need, chunk[k] + 1);
-                    } else {
-                        D.idx[at(4)] = ~k;
-                        far = 1;
-                    }
-                }
-            }
-            C.nblk = nblk | far << 8;
+            C.nblk = (most + SWEEP_BLK - 1) / SWEEP_BLK;
+            D.n_ent += (size_t)C.nblk * SWEEP_BLK * C.nr;
             D.chunks.push_back(C);
         }
 }
 
-int upload_side(rbfx_ctx* ctx, rbfx_stokes::Side& D, const HostSide& H) {
-    D.n_chunks = (int)H.chunks.size();
-    D.n_ent = (int)H.idx.size();
-    int rc;
-    if ((rc = upload(ctx, &D.chunks, H.chunks)) || (rc = upload(ctx, &D.rows, H.rows)) ||
-        (rc = upload(ctx, &D.idx, H.idx)) || (rc = upload(ctx, &D.src64, H.src64)) || (rc = upload(ctx, &D.src32, H.src32)))
-        return rc;
-    const size_t n = std::max<size_t>(1, H.idx.size());
-    if (hipMalloc((void**)&D.val64, n * sizeof(double)) != hipSuccess ||
-        (!H.src32.empty() && hipMalloc((void**)&D.val32, n * sizeof(float)) != hipSuccess))
-        return rbfx_fail(ctx, RBFX_E_NOMEM, "stokes_create: packed factor entries");
-    return RBFX_OK;
+// The error of the stencil at layout position p, which holds a node twice or misses its centre.
+int bad_stencil(rbfx_ctx* ctx, const rbfx_ell* ops, int p) {
+    const int W = ops->width;
+    int r = p;
+    std::vector<int32_t> c(W);
+    if (ops->order) RBFX_HIP_CHECK(ctx, hipMemcpy(&r, ops->order + p, sizeof(int32_t), hipMemcpyDeviceToHost));
+    for (int j = 0; j < W; j++)
+        RBFX_HIP_CHECK(ctx, hipMemcpy(&c[j], ops->idx_t + ell_row_base(p, W) + (size_t)j * ELL_TILE, sizeof(int32_t),
+                                      hipMemcpyDeviceToHost));
+    std::sort(c.begin(), c.end());
+    for (int j = 1; j < W; j++)
+        if (c[j] == c[j - 1])
+            return rbfx_fail(ctx, RBFX_E_INVALID, "stokes_create: stencil %d holds node %d twice", r, c[j]);
+    return rbfx_fail(ctx, RBFX_E_INVALID, "stokes_create: stencil %d does not contain its centre", r);
 }
 
 // y = A x (block layout, n_tot values) for the FP64 or FP32 operator set.
@@ -867,85 +935,7 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     const int N = ops64->n_rows, W = ops64->width;
     if (W > FACTOR_MAX_WIDTH) return rbfx_fail(ctx, RBFX_E_TOO_LARGE, "stokes_create: stencil width %d above %d", W, FACTOR_MAX_WIDTH);
     RBFX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
-    // the stencils and L weights back on the host, by row (layout position p holds row order[p])
-    const size_t tiles = (size_t)((N + ELL_TILE - 1) / ELL_TILE) * ELL_TILE * W;
-    std::vector<int32_t> idx_t(tiles), order(N);
-    std::vector<double> w_t(tiles * 4);
-    RBFX_HIP_CHECK(ctx, hipStreamSynchronize(ctx->stream));
-    RBFX_HIP_CHECK(ctx, hipMemcpy(idx_t.data(), ops64->idx_t, tiles * sizeof(int32_t), hipMemcpyDeviceToHost));
-    RBFX_HIP_CHECK(ctx, hipMemcpy(w_t.data(), ops64->w_t, tiles * 4 * sizeof(double), hipMemcpyDeviceToHost));
-    if (ops64->order)
-        RBFX_HIP_CHECK(ctx, hipMemcpy(order.data(), ops64->order, N * sizeof(int32_t), hipMemcpyDeviceToHost));
-    else
-        for (int i = 0; i < N; i++) order[i] = i;
-    // CSR of A_L = -eta L with each row's columns ascending (the reference's compressed_matrix)
-    std::vector<int32_t> ip(N + 1), col((size_t)N * W), dg(N);
-    std::vector<double> a((size_t)N * W);
-    std::vector<std::pair<int32_t, double>> ent(W);
-    for (int p = 0; p < N; p++) {
-        const int r = order[p];
-        const size_t base = ell_row_base(p, W);
-        for (int j = 0; j < W; j++) {
-            const size_t e = base + (size_t)j * ELL_TILE;
-            ent[j] = {idx_t[e], w_t[e * 4]};
-        }
-        std::sort(ent.begin(), ent.end(), [](const auto& x, const auto& y) { return x.first < y.first; });
-        int d = -1;
-        for (int j = 0; j < W; j++) {
-            if (j && ent[j].first == ent[j - 1].first)
-                return rbfx_fail(ctx, RBFX_E_INVALID, "stokes_create: stencil %d holds node %d twice", r, ent[j].first);
-            col[(size_t)r * W + j] = ent[j].first;
-            a[(size_t)r * W + j] = -eta * ent[j].second;
-            if (ent[j].first == r) d = j;
-        }
-        if (d < 0) return rbfx_fail(ctx, RBFX_E_INVALID, "stokes_create: stencil %d does not contain its centre", r);
-        dg[r] = r * W + d;
-    }
-    for (int r = 0; r <= N; r++) ip[r] = r * W;
-    // dependency levels: the lower sweep and the factorization read rows k < r of row r's
-    // pattern, the upper sweep rows k > r
-    std::vector<int32_t> lev(N, 0), ulev(N, 0);
-    int nl = 0, nu = 0;
-    for (int r = 0; r < N; r++) {
-        int m = -1;
-        for (int q = ip[r]; q < dg[r]; q++) m = std::max(m, lev[col[q]]);
-        lev[r] = m + 1;
-        nl = std::max(nl, m + 2);
-    }
-    for (int r = N - 1; r >= 0; r--) {
-        int m = -1;
-        for (int q = dg[r] + 1; q < ip[r + 1]; q++) m = std::max(m, ulev[col[q]]);
-        ulev[r] = m + 1;
-        nu = std::max(nu, m + 2);
-    }
-    auto by_level = [&](const std::vector<int32_t>& L, int n_lev, std::vector<int32_t>& rows, std::vector<int32_t>& off) {
-        off.assign(n_lev + 1, 0);
-        for (int r = 0; r < N; r++) off[L[r] + 1]++;
-        for (int l = 0; l < n_lev; l++) off[l + 1] += off[l];
-        rows.assign(N, 0);
-        std::vector<int32_t> pos(off.begin(), off.end() - 1);
-        for (int r = 0; r < N; r++) rows[pos[L[r]]++] = r;
-    };
-    int max_side = 0;
-    for (int r = 0; r < N; r++) max_side = std::max({max_side, dg[r] - ip[r], ip[r + 1] - dg[r] - 1});
-    std::vector<int32_t> lrows, loff, urows, uoff;
-    by_level(lev, nl, lrows, loff);
-    by_level(ulev, nu, urows, uoff);
-    const int nb = sweep_variant((max_side + SWEEP_BLK - 1) / SWEEP_BLK);
-    HostSide low, up;
-    const bool fp32 = ops32 != nullptr;  // the FP32 copy of the factor serves the FP32 inner solves
-    pack_side(lrows, loff, N, nb, false, fp32, low, [&](int r, int& a, int& b) { a = ip[r], b = dg[r]; }, col);
-    pack_side(urows, uoff, N, nb, true, fp32, up, [&](int r, int& a, int& b) { a = dg[r] + 1, b = ip[r + 1]; }, col);
-    std::vector<int32_t> uds(N);
-    for (int t = 0; t < N; t++) uds[t] = dg[urows[t]];
-    // what rbfx_stokes_info reports: levels in steps of at most 32 rows (16 for wide stencils)
-    const int slots = max_side > 32 ? 16 : 32;
-    auto steps = [&](const std::vector<int32_t>& off) {
-        int n = 0;
-        for (size_t l = 0; l + 1 < off.size(); l++) n += (off[l + 1] - off[l] + slots - 1) / slots;
-        return n;
-    };
-
+    hipStream_t st = ctx->stream;
     rbfx_stokes* S = new rbfx_stokes();
     S->ctx = ctx;
     S->e64 = ops64;
@@ -954,50 +944,128 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     S->N = N;
     S->width = W;
     S->n_tot = 4 * (size_t)N + 4;
-    S->n_lev_l = steps(loff);
-    S->n_lev_u = steps(uoff);
-    S->nb = nb;
-    int rc = RBFX_OK;
-    if ((rc = upload(ctx, &S->col, col)) || (rc = upload(ctx, &S->diag, dg)) || (rc = upload(ctx, &S->a_in, a)) ||
-        (rc = upload_side(ctx, S->low, low)) || (rc = upload_side(ctx, S->up, up)) ||
-        (rc = upload(ctx, &S->udsrc, uds)) || (rc = workspace(S, 1))) {
+    auto fail = [&](int code, const char* what, hipError_t err) {
+        hipStreamSynchronize(st);
+        stokes_free(S);
+        delete S;
+        return rbfx_fail(ctx, code, "stokes_create: %s: %s", what, hipGetErrorString(err));
+    };
+    const size_t nnz = (size_t)N * W;
+    auto carve_rows = [&](Carver& m) {
+        m.take(&S->col, nnz);
+        m.take(&S->diag, N);
+        m.take(&S->a_in, nnz);
+        m.take(&S->f64, nnz);
+        m.take(&S->counter, 1);
+        m.take(&S->err, 1);
+        m.take(&S->low.rows, N);  // the factorization's order too
+    };
+    Carver rows_mem;
+    carve_rows(rows_mem);
+    hipError_t e = hipMalloc(&S->rows_mem, rows_mem.used);
+    if (e != hipSuccess) return fail(RBFX_E_NOMEM, "matrix and factor", e);
+    rows_mem = Carver{(unsigned char*)S->rows_mem};
+    carve_rows(rows_mem);
+    // A_L by rows on the device; its pattern comes back for the dependency levels
+    factor_init_kernel<<<blocks_for(nnz, 256), 256, 0, st>>>((unsigned long long*)S->f64, nnz, S->counter, S->err);
+    stokes_rows_kernel<<<blocks_for(N, 4), 256, 0, st>>>(ops64->idx_t, (const double*)ops64->w_t, ops64->order, N, W, eta, S->col,
+                                                        S->a_in, S->diag, S->err);
+    std::vector<int32_t> col(nnz), dg(N);
+    int bad = 0;
+    if ((e = hipGetLastError()) != hipSuccess ||
+        (e = hipMemcpyAsync(col.data(), S->col, nnz * sizeof(int32_t), hipMemcpyDeviceToHost, st)) != hipSuccess ||
+        (e = hipMemcpyAsync(dg.data(), S->diag, N * sizeof(int32_t), hipMemcpyDeviceToHost, st)) != hipSuccess ||
+        (e = hipMemcpyAsync(&bad, S->err, sizeof(int), hipMemcpyDeviceToHost, st)) != hipSuccess ||
+        (e = hipStreamSynchronize(st)) != hipSuccess)
+        return fail(RBFX_E_HIP, "assembly", e);
+    if (bad < N) {
+        stokes_free(S);
+        delete S;
+        return bad_stencil(ctx, ops64, bad);
+    }
+    // dependency levels: the lower sweep and the factorization read rows k < r of row r's
+    // pattern, the upper sweep rows k > r (found while the factorization runs)
+    std::vector<int32_t> lev(N);
+    int n_lev = 0, max_side = 0;
+    for (int r = 0; r < N; r++) {
+        int m = -1;
+        for (int q = r * W; q < dg[r]; q++) m = std::max(m, lev[col[q]]);
+        lev[r] = m + 1;
+        n_lev = std::max(n_lev, m + 2);
+        max_side = std::max({max_side, dg[r] - r * W, (r + 1) * W - dg[r] - 1});
+    }
+    HostSide low, up;
+    order_side(lev, n_lev, [&](int r) { return dg[r] - r * W; }, low);
+    auto send = [&](auto* d, const auto& h) {
+        if (e == hipSuccess) e = hipMemcpyAsync(d, h.data(), h.size() * sizeof(h[0]), hipMemcpyHostToDevice, st);
+    };
+    send(S->low.rows, low.rows);
+    if (e == hipSuccess) {
+        ilu0_factor_kernel<<<FACTOR_BLOCKS, 64 * FACTOR_WAVES, 0, st>>>(S->col, S->diag, S->a_in, S->low.rows, N, W, S->counter,
+                                                                       S->f64);
+        e = hipGetLastError();
+    }
+    if (e != hipSuccess) return fail(RBFX_E_HIP, "ILU(0) factorization", e);
+    n_lev = 0;
+    for (int r = N - 1; r >= 0; r--) {
+        int m = -1;
+        for (int q = dg[r] + 1; q < (r + 1) * W; q++) m = std::max(m, lev[col[q]]);
+        lev[r] = m + 1;
+        n_lev = std::max(n_lev, m + 2);
+    }
+    order_side(lev, n_lev, [&](int r) { return (r + 1) * W - dg[r] - 1; }, up);
+    S->nb = sweep_variant((max_side + SWEEP_BLK - 1) / SWEEP_BLK);
+    // what rbfx_stokes_info reports: levels in steps of at most 32 rows (16 for wide stencils)
+    const int slots = max_side > 32 ? 16 : 32;
+    auto steps = [&](const std::vector<int32_t>& off) {
+        int n = 0;
+        for (size_t l = 0; l + 1 < off.size(); l++) n += (off[l + 1] - off[l] + slots - 1) / slots;
+        return n;
+    };
+    S->n_lev_l = steps(low.off);
+    S->n_lev_u = steps(up.off);
+    const bool fp32 = ops32 != nullptr;  // the FP32 copy of the factor serves the FP32 inner solves
+    auto carve_sweeps = [&](Carver& m) {
+        for (auto [D, H] : {std::pair{&S->low, &low}, std::pair{&S->up, &up}}) {
+            D->n_chunks = (int)H->chunks.size();
+            m.take(&D->chunks, H->chunks.size());
+            if (D == &S->up) m.take(&D->rows, N);
+            m.take(&D->task, N);
+            m.take(&D->chunk_of, N);
+            m.take(&D->idx, H->n_ent);
+            m.take(&D->val64, H->n_ent);
+            if (fp32) m.take(&D->val32, H->n_ent);
+        }
+        m.take(&S->ud64, N);
+        if (fp32) m.take(&S->ud32, N);
+    };
+    Carver sweep_mem;
+    carve_sweeps(sweep_mem);
+    if ((e = hipMalloc(&S->sweep_mem, sweep_mem.used)) != hipSuccess) return fail(RBFX_E_NOMEM, "packed factor entries", e);
+    sweep_mem = Carver{(unsigned char*)S->sweep_mem};
+    carve_sweeps(sweep_mem);
+    const int rc = workspace(S, 1);
+    if (rc) {
+        hipStreamSynchronize(st);
         stokes_free(S);
         delete S;
         return rc;
     }
-    if (hipMalloc((void**)&S->f64, (size_t)N * W * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&S->counter, sizeof(int)) != hipSuccess ||
-        hipMalloc((void**)&S->ud64, N * sizeof(double)) != hipSuccess || hipMalloc((void**)&S->ud32, N * sizeof(float)) != hipSuccess) {
-        stokes_free(S);
-        delete S;
-        return rbfx_fail(ctx, RBFX_E_NOMEM, "stokes_create: packed factor entries");
-    }
-    hipError_t e = hipSuccess;
-    if (e == hipSuccess) {
-        const size_t nnz = (size_t)N * W;
-        factor_init_kernel<<<blocks_for(nnz, 256), 256, 0, ctx->stream>>>((unsigned long long*)S->f64, nnz, S->counter);
-        ilu0_factor_kernel<<<FACTOR_BLOCKS, 64 * FACTOR_WAVES, 0, ctx->stream>>>(S->col, S->diag, S->a_in, S->low.rows, N, W,
-                                                                                S->counter, S->f64);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) {
-        hipStream_t st = ctx->stream;
-        for (rbfx_stokes::Side* D : {&S->low, &S->up}) {
-            if (!D->n_ent) continue;
-            gather_kernel<double><<<blocks_for(D->n_ent, 256), 256, 0, st>>>(S->f64, D->src64, D->val64, D->n_ent);
-            if (D->val32)
-                gather_kernel<float><<<blocks_for(D->n_ent, 256), 256, 0, st>>>(S->f64, D->src32, D->val32, D->n_ent);
+    for (auto [D, H] : {std::pair{&S->low, &low}, std::pair{&S->up, &up}}) {
+        const bool upper = D == &S->up;
+        send(D->chunks, H->chunks);
+        if (upper) send(D->rows, H->rows);
+        send(D->task, H->task);
+        send(D->chunk_of, H->chunk_of);
+        if (e == hipSuccess) {
+            pack_sweep_kernel<<<blocks_for(D->n_chunks, 4), 256, 0, st>>>(D->chunks, D->n_chunks, D->rows, D->task, D->chunk_of,
+                                                                         S->col, S->diag, S->f64, W, S->nb, upper, D->idx,
+                                                                         D->val64, D->val32, upper ? S->ud64 : nullptr, S->ud32);
+            e = hipGetLastError();
         }
-        gather_kernel<double><<<blocks_for(N, 256), 256, 0, st>>>(S->f64, S->udsrc, S->ud64, N);
-        gather_kernel<float><<<blocks_for(N, 256), 256, 0, st>>>(S->f64, S->udsrc, S->ud32, N);
-        e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    if (e != hipSuccess) {
-        stokes_free(S);
-        delete S;
-        return rbfx_fail(ctx, RBFX_E_HIP, "stokes_create: ILU(0) factorization: %s", hipGetErrorString(e));
-    }
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return fail(RBFX_E_HIP, "ILU(0) factorization", e);
     *out = S;
     return RBFX_OK;
 }
