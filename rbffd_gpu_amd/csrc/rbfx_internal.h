@@ -53,4 +53,15 @@ int rbfx_fail(rbfx_ctx* ctx, int code, const char* fmt, ...);
                              hipGetErrorString(e_));                                          \
     } while (0)
 
+// Pieces of one allocation, each on 256 bytes: carve once without memory for the size, then with it.
+struct Carver {
+    unsigned char* base = nullptr;
+    size_t used = 0;
+    template <typename T>
+    void take(T** p, size_t n) {
+        if (base) *p = reinterpret_cast<T*>(base + used);
+        used += (n * sizeof(T) + 255) / 256 * 256;
+    }
+};
+
 static inline unsigned popcount32(uint32_t x) { return (unsigned)__builtin_popcount(x); }

@@ -8,17 +8,17 @@
 // the tree visits them in. Only when two of those k+1 distances are equal do the heap's sift
 // rules and the visit order decide which point comes first (or which of two equidistant
 // points at the k-th place is kept). So:
-//   * the GPU runs an exact search over a uniform grid of cubic cells, one query per thread,
-//     keeping the k+1 best (distance, id) pairs in LDS in ascending order;
+//   * the GPU runs an exact search over a uniform grid of cubic cells, one query per wave;
 //   * distances are computed exactly as the kd-tree does, (q0-p0)^2 + (q1-p1)^2 + (q2-p2)^2
 //     summed left to right with every product and sum rounded on its own (no fused
 //     multiply-add), so equal inputs give equal keys on both sides;
 //   * a query whose k+1 best distances are not strictly increasing is handed back and
 //     recomputed on the host by the kd-tree (rbfx_knn_kdtree_rows).
-// The search visits cells in shells of growing Chebyshev radius r around the query's cell;
-// every point outside the cells visited so far is at least r * h away, so the search stops
-// once the (k+1)-th best distance is below (r h)^2 (with a 1e-9 relative margin for the
-// rounding of cell assignment and distances), and at the latest when r covers the grid.
+//
+// The grid is built on the device too: bounding box, the number of occupied cells at halved cell
+// sizes, the cell size between two of them at which a ball of its radius holds a little more than
+// k+1 nodes, and a counting sort of the nodes by cell. (rbfx_knn_grid_bin in csrc/rbfx_knn.cpp
+// states such a binning on the host.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -28,95 +28,431 @@
 #include <cstring>
 #include <vector>
 
+#include "rbfx_ell_common.h"
 #include "rbfx_host_internal.h"
-#include "rbfx_internal.h"
 
 namespace {
 
-struct KnnArgs {
-    const double* pts;      // points sorted by cell, xyz interleaved
-    const int32_t* pid;     // node id of each sorted point
-    const int32_t* cstart;  // cell c holds sorted points cstart[c] .. cstart[c+1]
-    const double* q;        // query coordinates (the nodes, in node order)
-    int32_t* out;           // n x k neighbour ids
-    int32_t* flag;          // 1: distance tie among the k+1 best, recompute on the host
-    int n, k, gx, gy, gz;
-    double lo0, lo1, lo2, inv_h, h;
+constexpr int KNN_CAP = 256;        // candidates a wave ranks
+constexpr int KNN_MAX_K1 = 170;     // longer lists are left to the host kd-tree
+constexpr int KNN_WAVES = 4;        // per workgroup
+constexpr int KNN_PER_WAVE = 8;     // queries of a wave, one after the other
+constexpr int KNN_LEVELS = 11;      // halvings of the cell size that are counted
+constexpr int BOUND_BLOCKS = 256;
+constexpr int SCAN_THREADS = 256, SCAN_PER = 16, SCAN_TILE = SCAN_THREADS * SCAN_PER;
+
+struct Point {
+    double x, y, z;
+    int id, pad;
 };
 
-__device__ __forceinline__ int cell_of(double x, double lo, double inv_h, int g) {
+struct Grid {
+    double lo[3], h, inv_h;
+    int g[3];
+    int n_cells;
+};
+
+struct Plan {
+    Grid grid;
+    double lo[3], hi[3];
+    int bad;     // a coordinate is not finite
+    int n_ties;  // rows handed back
+    // occupancy levels: grids of halved cells and where their cells' bytes start
+    int n_levels;
+    Grid level[KNN_LEVELS];
+    int cell0[KNN_LEVELS + 1];
+    int occupied[KNN_LEVELS];
+};
+
+__device__ __forceinline__ int cell_coord(double x, double lo, double inv_h, int g) {
     const int c = (int)((x - lo) * inv_h);  // x >= lo
     return c < 0 ? 0 : (c >= g ? g - 1 : c);
 }
 
-// One query per thread; the sorted k+1 best live in LDS at [slot * B + thread].
-__global__ void __launch_bounds__(64) knn_grid_kernel(KnnArgs a) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const int B = blockDim.x, t = threadIdx.x, K1 = a.k + 1;
-    double* dl = reinterpret_cast<double*>(smem);
-    int* il = reinterpret_cast<int*>(dl + (size_t)K1 * B);
-    const int i = blockIdx.x * B + t;
-    if (i >= a.n) return;  // the kernel has no barriers
-    const double q0 = a.q[3 * (size_t)i], q1 = a.q[3 * (size_t)i + 1], q2 = a.q[3 * (size_t)i + 2];
-    const int cx = cell_of(q0, a.lo0, a.inv_h, a.gx), cy = cell_of(q1, a.lo1, a.inv_h, a.gy),
-              cz = cell_of(q2, a.lo2, a.inv_h, a.gz);
-    const int rmax = max(a.gx, max(a.gy, a.gz));  // at rmax every cell has been visited
-    int cnt = 0;
-    for (int r = 0; r <= rmax; r++) {
-        for (int dz = -r; dz <= r; dz++) {
-            const int z = cz + dz;
-            if (z < 0 || z >= a.gz) continue;
-            for (int dy = -r; dy <= r; dy++) {
-                const int y = cy + dy;
-                if (y < 0 || y >= a.gy) continue;
-                // on the shell's faces every dx; inside it only dx = -r and dx = +r
-                const int step = (dz == -r || dz == r || dy == -r || dy == r || r == 0) ? 1 : 2 * r;
-                for (int dx = -r; dx <= r; dx += step) {
-                    const int x = cx + dx;
-                    if (x < 0 || x >= a.gx) continue;
-                    const size_t c = ((size_t)z * a.gy + y) * a.gx + x;
-                    const int s1 = a.cstart[c + 1];
-                    for (int s = a.cstart[c]; s < s1; s++) {
-                        const double e0 = q0 - a.pts[3 * (size_t)s], e1 = q1 - a.pts[3 * (size_t)s + 1],
-                                     e2 = q2 - a.pts[3 * (size_t)s + 2];
-                        const double d = dadd_nc(dadd_nc(dmul_nc(e0, e0), dmul_nc(e1, e1)), dmul_nc(e2, e2));
-                        int pos;
-                        if (cnt < K1) {
-                            pos = cnt++;
-                        } else if (d < dl[(size_t)(K1 - 1) * B + t]) {
-                            pos = K1 - 1;
-                        } else {
-                            continue;
+__device__ __forceinline__ int cell_index(const Grid& G, double x, double y, double z) {
+    return (cell_coord(z, G.lo[2], G.inv_h, G.g[2]) * G.g[1] + cell_coord(y, G.lo[1], G.inv_h, G.g[1])) * G.g[0] +
+           cell_coord(x, G.lo[0], G.inv_h, G.g[0]);
+}
+
+// Cells of size h over a box; false when they number more than max_cells.
+__device__ bool set_cells(Grid& G, const double* lo, const double* hi, double h, int max_cells) {
+    double total = 1.0;
+    G.h = h;
+    G.inv_h = 1.0 / h;
+    for (int d = 0; d < 3; d++) {
+        G.lo[d] = lo[d];
+        const double c = floor((hi[d] - lo[d]) * G.inv_h) + 1.0;
+        G.g[d] = c < 1.0 ? 1 : (c > 1e6 ? 1000000 : (int)c);
+        total *= G.g[d];
+    }
+    G.n_cells = total <= (double)max_cells ? (int)total : 0;
+    return G.n_cells > 0;
+}
+
+// Per block: the box of its nodes, lo and hi, and whether a coordinate is not finite.
+__global__ void __launch_bounds__(256) knn_bounds_kernel(const double* __restrict__ xyz, int n, double* __restrict__ part) {
+    __shared__ double s[256][7];
+    double v[7] = {DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX, 0.0};
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < (size_t)n; i += (size_t)gridDim.x * 256)
+        for (int d = 0; d < 3; d++) {
+            const double c = xyz[3 * i + d];
+            v[6] = isfinite(c) ? v[6] : 1.0;
+            v[d] = fmin(v[d], c);
+            v[3 + d] = fmax(v[3 + d], c);
+        }
+    for (int q = 0; q < 7; q++) s[threadIdx.x][q] = v[q];
+    for (int o = 128; o > 0; o >>= 1) {
+        __syncthreads();
+        if (threadIdx.x < o)
+            for (int q = 0; q < 7; q++) {
+                const double a = s[threadIdx.x][q], b = s[threadIdx.x + o][q];
+                s[threadIdx.x][q] = q < 3 ? fmin(a, b) : fmax(a, b);
+            }
+    }
+    if (threadIdx.x == 0)
+        for (int q = 0; q < 7; q++) part[blockIdx.x * 7 + q] = s[0][q];
+}
+
+// The box of all nodes and the levels whose cells are counted: the largest extent cut into 4, 8,
+// 16, ... cells, as long as they number at most max_cells.
+__global__ void __launch_bounds__(64) knn_levels_kernel(const double* __restrict__ part, int n_part, int max_cells, Plan* P) {
+    double lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX}, bad = 0.0;
+    for (int b = threadIdx.x; b < n_part; b += 64) {
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], part[b * 7 + d]);
+            hi[d] = fmax(hi[d], part[b * 7 + 3 + d]);
+        }
+        bad = fmax(bad, part[b * 7 + 6]);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        for (int d = 0; d < 3; d++) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], o));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], o));
+        }
+        bad = fmax(bad, __shfl_xor(bad, o));
+    }
+    if (threadIdx.x) return;
+    P->bad = bad != 0.0;
+    P->n_ties = 0;
+    for (int d = 0; d < 3; d++) {
+        P->lo[d] = lo[d];
+        P->hi[d] = hi[d];
+    }
+    double ext = fmax(hi[0] - lo[0], fmax(hi[1] - lo[1], hi[2] - lo[2]));
+    if (!(ext > 0.0) || !isfinite(ext)) ext = 1.0;
+    int l = 0, cell = 0;
+    for (; l < KNN_LEVELS; l++) {
+        // the bytes of all levels share max_cells
+        if (!set_cells(P->level[l], lo, hi, ext * (1.0 + 1e-12) / (double)(4 << l), max_cells - cell - 4)) break;
+        P->cell0[l] = cell;
+        P->occupied[l] = 0;
+        cell += (P->level[l].n_cells + 3) / 4 * 4;
+    }
+    P->n_levels = l;
+    P->cell0[l] = cell;
+}
+
+// A byte per cell of every level, set by plain stores: all of them store the same 1. (Bits set by
+// atomic or took 7.8 ms for a million nodes in a locality order, whose words many waves share.)
+__global__ void __launch_bounds__(256) knn_mark_kernel(const double* __restrict__ xyz, int n, const Plan* __restrict__ P,
+                                                      uint8_t* seen) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)n || P->bad) return;
+    const double x = xyz[3 * i], y = xyz[3 * i + 1], z = xyz[3 * i + 2];
+    for (int l = 0; l < P->n_levels; l++) {
+        const int c = P->cell0[l] + cell_index(P->level[l], x, y, z);
+        if (!seen[c]) seen[c] = 1;
+    }
+}
+
+// blockIdx.y: level
+__global__ void __launch_bounds__(256) knn_occupied_kernel(Plan* P, const uint8_t* __restrict__ seen) {
+    const int l = blockIdx.y;
+    if (l >= P->n_levels) return;
+    const unsigned* words = reinterpret_cast<const unsigned*>(seen);  // levels start at multiples of 4, bytes past them are 0
+    int c = 0;
+    for (int w = P->cell0[l] / 4 + blockIdx.x * 256 + threadIdx.x; w < P->cell0[l + 1] / 4; w += gridDim.x * 256) c += __popc(words[w]);
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+    if (threadIdx.x % 64 == 0 && c) atomicAdd(&P->occupied[l], c);
+}
+
+// The cell size at which an occupied cell holds 0.29 (k+1) nodes, between the two levels around
+// it: on a surface a ball of that radius then holds about 1.35 (k+1) nodes (a plane meets 1.5 cells
+// per cell area on average, so the ball covers 1.5 pi of them), in a volume 1.2 (k+1). Mostly the
+// 27 cells around a query then answer it, with one or two candidates per lane.
+__global__ void knn_choose_kernel(Plan* P, int n, int k, int max_cells) {
+    if (threadIdx.x || blockIdx.x || P->bad) return;
+    const double want = fmax(1.5, 0.29 * (k + 1));
+    double h = P->n_levels ? P->level[0].h : 1.0, above = 0.0;  // above: nodes per occupied cell one level up
+    for (int l = 0; l < P->n_levels; l++) {
+        const double per = (double)n / (double)max(1, P->occupied[l]);
+        h = P->level[l].h;
+        if (per <= want) {
+            if (l > 0 && above > per) h *= exp2(log(want / per) / log(above / per));
+            break;
+        }
+        above = per;
+    }
+    for (int it = 0; it < 64; it++, h *= 1.25)
+        if (set_cells(P->grid, P->lo, P->hi, h, max_cells)) return;
+    // no such size (the box's extent overflows): one cell, which every search covers at once
+    P->grid = Grid{{P->lo[0], P->lo[1], P->lo[2]}, 1.0, 0.0, {1, 1, 1}, 1};
+}
+
+__global__ void __launch_bounds__(256) knn_count_kernel(const double* __restrict__ xyz, int n, const Plan* __restrict__ P,
+                                                       int* __restrict__ count) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < (size_t)n) atomicAdd(&count[cell_index(P->grid, xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2])], 1);
+}
+
+// Exclusive prefix sums: tiles of SCAN_TILE counts, then the tiles' totals (one block), then both.
+__global__ void __launch_bounds__(SCAN_THREADS) knn_scan_kernel(const int* __restrict__ count, int n, int* __restrict__ start,
+                                                               int* __restrict__ total) {
+    __shared__ int s[SCAN_THREADS / 64];
+    const int t = threadIdx.x, lane = t % 64;
+    const int i0 = blockIdx.x * SCAN_TILE + t * SCAN_PER;
+    int v[SCAN_PER], sum = 0;
+#pragma unroll
+    for (int q = 0; q < SCAN_PER; q++) {
+        v[q] = sum;
+        sum += i0 + q < n ? count[i0 + q] : 0;
+    }
+    int in = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(in, o);
+        if (lane >= o) in += up;
+    }
+    if (lane == 63) s[t / 64] = in;
+    __syncthreads();
+    int before = in - sum;
+    for (int w = 0; w < t / 64; w++) before += s[w];
+#pragma unroll
+    for (int q = 0; q < SCAN_PER; q++)
+        if (i0 + q < n) start[i0 + q] = before + v[q];
+    if (t == SCAN_THREADS - 1) total[blockIdx.x] = before + sum;
+}
+
+__global__ void __launch_bounds__(1024) knn_scan_totals_kernel(int* __restrict__ total, int n) {
+    __shared__ int s[16];
+    const int t = threadIdx.x, lane = t % 64;
+    int carry = 0;
+    for (int i0 = 0; i0 < n; i0 += 1024) {
+        const int v = i0 + t < n ? total[i0 + t] : 0;
+        int in = v;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int up = __shfl_up(in, o);
+            if (lane >= o) in += up;
+        }
+        if (lane == 63) s[t / 64] = in;
+        __syncthreads();
+        int before = carry, all = 0;
+        for (int w = 0; w < 16; w++) {
+            if (w < t / 64) before += s[w];
+            all += s[w];
+        }
+        if (i0 + t < n) total[i0 + t] = before + in - v;
+        carry += all;
+        __syncthreads();
+    }
+}
+
+__global__ void __launch_bounds__(256) knn_scan_add_kernel(int* __restrict__ start, int n, const int* __restrict__ total,
+                                                          int n_points) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) start[i] += total[i / SCAN_TILE];
+    if (i == n) start[n] = n_points;
+}
+
+// Every node into its cell's run; the order inside a cell does not matter to the search.
+__global__ void __launch_bounds__(256) knn_scatter_kernel(const double* __restrict__ xyz, int n, const Plan* __restrict__ P,
+                                                         const int* __restrict__ start, int* __restrict__ count,
+                                                         Point* __restrict__ pts) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (size_t)n) return;
+    const Point p = {xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], (int)i, 0};
+    const int c = cell_index(P->grid, p.x, p.y, p.z);
+    pts[start[c] + atomicSub(&count[c], 1) - 1] = p;
+}
+
+struct KnnArgs {
+    const Point* pts;   // nodes sorted by cell
+    const int* start;   // cell c holds pts[start[c]] .. pts[start[c + 1]]
+    Plan* plan;
+    int32_t* out;       // n x k neighbour ids
+    int32_t* ties;      // rows with a distance tie among their k+1 best
+    int n, k, nb;
+};
+
+// One query per wave at a time, queries in cell order. All nodes in the cells within Chebyshev distance r of
+// the query's are looked at, and those closer than r * h (with a 1e-9 relative margin for the rounding
+// of cell assignment and distances; every other node is farther) are kept in LDS. Fewer than k+1:
+// r grows. More than KNN_CAP: the bound is narrowed until between k+1 and KNN_CAP are kept. They hold the
+// k+1 best; the place of each is the number of closer ones. The cells of a row along x are one run of
+// sorted nodes: quarter waves take a run each.
+//
+// Bound: instruction issue, about 200 candidates and 70 x 70 compared distances a query. N = 10^6, k = 50:
+// 1.14 ms; a query per thread with a sorted list of k+1 in LDS (four waves per CU, 130 insertions of
+// 25 moves each) took 11.3 ms. The grid kernels take 0.2 ms; binning on the host, with its copies,
+// took 27 ms of a call of 41-50 ms, which now takes 2.6 ms.
+__global__ void __launch_bounds__(64 * KNN_WAVES) knn_grid_kernel(KnnArgs a) {
+    __shared__ double s_d[KNN_WAVES][KNN_CAP];
+    __shared__ int s_id[KNN_WAVES][KNN_CAP];
+    __shared__ int s_out[KNN_WAVES][KNN_CAP];
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    double(&D)[KNN_CAP] = s_d[wave];
+    int(&ID)[KNN_CAP] = s_id[wave];
+    int(&OUT)[KNN_CAP] = s_out[wave];
+    auto wave_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    const Grid G = a.plan->grid;
+    const int K1 = a.k + 1, g_max = max(G.g[0], max(G.g[1], G.g[2]));
+    const long long q0 = ((long long)xcd_tile(blockIdx.x, a.nb) * KNN_WAVES + wave) * KNN_PER_WAVE;
+    for (long long s = q0; s < q0 + KNN_PER_WAVE && s < a.n; s++) {
+        const Point q = a.pts[s];
+        const int cx = cell_coord(q.x, G.lo[0], G.inv_h, G.g[0]), cy = cell_coord(q.y, G.lo[1], G.inv_h, G.g[1]),
+                  cz = cell_coord(q.z, G.lo[2], G.inv_h, G.g[2]);
+        // keeps the nodes within r cells that are closer than bound (or all); returns how many there are
+        auto collect = [&](int r, double bound, bool all) {
+            int kept = 0;
+            const int x0 = max(cx - r, 0), x1 = min(cx + r, G.g[0] - 1);
+            const int y0 = max(cy - r, 0), ny = min(cy + r, G.g[1] - 1) - y0 + 1;
+            const int z0 = max(cz - r, 0), nz = min(cz + r, G.g[2] - 1) - z0 + 1;
+            for (int c0 = 0; c0 < ny * nz; c0 += 64) {
+                const int j = c0 + lane;
+                int p0 = 0, p1 = 0;
+                if (j < ny * nz) {
+                    const int row = ((z0 + j / ny) * G.g[1] + y0 + j % ny) * G.g[0];
+                    p0 = a.start[row + x0];
+                    p1 = a.start[row + x1 + 1];
+                }
+                unsigned long long runs = __ballot(p1 > p0);
+                while (runs) {
+                    int run[4];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        run[u] = runs ? __ffsll(runs) - 1 : -1;
+                        runs &= runs - 1;
+                    }
+                    const int u = lane / 16;
+                    const int mine = u == 0 ? run[0] : u == 1 ? run[1] : u == 2 ? run[2] : run[3];
+                    int p = __shfl(p0, max(mine, 0));
+                    const int last = __shfl(p1, max(mine, 0));  // by every lane: a shuffle reads active lanes only
+                    const int end = mine < 0 ? p : last;
+                    for (p += lane % 16; __any(p < end); p += 16) {
+                        double d = 0.0;
+                        int id = 0;
+                        bool keep = false;
+                        if (p < end) {
+                            const Point o = a.pts[p];
+                            const double e0 = q.x - o.x, e1 = q.y - o.y, e2 = q.z - o.z;
+                            d = dadd_nc(dadd_nc(dmul_nc(e0, e0), dmul_nc(e1, e1)), dmul_nc(e2, e2));
+                            id = o.id;
+                            keep = all || d < bound;
                         }
-                        while (pos > 0 && dl[(size_t)(pos - 1) * B + t] > d) {
-                            dl[(size_t)pos * B + t] = dl[(size_t)(pos - 1) * B + t];
-                            il[(size_t)pos * B + t] = il[(size_t)(pos - 1) * B + t];
-                            pos--;
+                        const unsigned long long m = __ballot(keep);
+                        const int at = kept + __popcll(m & ((1ull << lane) - 1));
+                        if (keep && at < KNN_CAP) {
+                            D[at] = d;
+                            ID[at] = id;
                         }
-                        dl[(size_t)pos * B + t] = d;
-                        il[(size_t)pos * B + t] = a.pid[s];
+                        kept += __popcll(m);
                     }
                 }
             }
+            wave_sync();
+            return kept;
+        };
+        wave_sync();  // the last query's lists have been read
+        int n_c = 0, n_lo = 0, r = 1;
+        double lo = 0.0, bound = 0.0;
+        bool all = false;
+        for (;;) {
+            all = r >= g_max;  // every cell is covered
+            bound = (double)r * G.h;
+            bound = bound * bound * (1.0 - 1e-9);
+            n_c = collect(r, bound, all);
+            if (n_c >= K1 || all) break;
+            lo = bound;
+            n_lo = n_c;
+            r += max(1, r / 2);
         }
-        if (cnt == K1) {
-            const double bound = (double)r * a.h;
-            if (dl[(size_t)(K1 - 1) * B + t] < bound * bound * (1.0 - 1e-9)) break;
+        if (n_c > KNN_CAP) {
+            // the number of nodes is about linear in the squared distance on a surface; with all nodes
+            // taken, the largest distance in the box bounds it
+            double hi = bound;
+            if (all) {
+                hi = 0.0;
+                for (int d = 0; d < 3; d++) hi += (a.plan->hi[d] - a.plan->lo[d]) * (a.plan->hi[d] - a.plan->lo[d]);
+                hi *= 1.0 + 1e-9;
+            }
+            double n_hi = n_c;
+            for (int it = 0; it < 100 && (n_c < K1 || n_c > KNN_CAP); it++) {
+                double part = (0.5 * (K1 + KNN_CAP) - n_lo) / (n_hi - n_lo);
+                part = it % 2 ? 0.5 : fmin(fmax(part, 0.02), 0.98);
+                bound = lo + (hi - lo) * part;
+                n_c = collect(r, bound, false);
+                if (n_c < K1) {
+                    lo = bound;
+                    n_lo = n_c;
+                } else {
+                    hi = bound;
+                    n_hi = n_c;
+                }
+            }
         }
+        bool tie = n_c < K1 || n_c > KNN_CAP;  // no bound found: many nodes at one distance
+        if (tie && n_lo == a.k) {              // it is the (k+1)-th distance: the k below it are the list
+            n_c = collect(r, lo, false);
+            tie = n_c != a.k;
+        }
+        const int i = q.id;
+        if (!tie) {
+            int place[KNN_CAP / 64];
+#pragma unroll
+            for (int c = 0; c < KNN_CAP / 64; c++) {
+                place[c] = KNN_CAP;
+                if (c * 64 < n_c) {
+                    const int j = c * 64 + lane;
+                    const double d = j < n_c ? D[j] : DBL_MAX;
+                    int closer = 0;
+                    for (int m = 0; m < n_c; m++) closer += D[m] < d;
+                    if (j < n_c && closer < a.k) {
+                        place[c] = closer;
+                        OUT[closer] = j;
+                    }
+                }
+            }
+            wave_sync();
+            // equal distances share a place: all but one of them find another candidate there
+#pragma unroll
+            for (int c = 0; c < KNN_CAP / 64; c++)
+                if (c * 64 < n_c) tie |= place[c] < a.k && OUT[place[c]] != c * 64 + lane;
+            tie = __any(tie);
+            if (!tie)
+                for (int t = lane; t < a.k; t += 64) a.out[(size_t)i * a.k + t] = ID[OUT[t]];
+        }
+        if (tie && lane == 0) a.ties[atomicAdd(&a.plan->n_ties, 1)] = i;
     }
-    int tie = 0;
-    for (int j = 0; j < a.k; j++) tie |= dl[(size_t)j * B + t] == dl[(size_t)(j + 1) * B + t];
-    a.flag[i] = tie;
-    for (int j = 0; j < a.k; j++) a.out[(size_t)i * a.k + j] = il[(size_t)j * B + t];
 }
 
-struct DevBufs {
-    void* p[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-    ~DevBufs() {
-        for (void* q : p)
-            if (q) hipFree(q);
+// Rows of k entries from the host to their places.
+__global__ void __launch_bounds__(256) knn_put_rows_kernel(const int32_t* __restrict__ rows, const int32_t* __restrict__ val, int n,
+                                                          int k, int32_t* __restrict__ out) {
+    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (e < (size_t)n * k) out[(size_t)rows[e / k] * k + e % k] = val[e];
+}
+
+struct DevBuf {
+    void* p = nullptr;
+    ~DevBuf() {
+        if (p) hipFree(p);
     }
 };
+
+unsigned blocks_for(size_t n, size_t per) { return (unsigned)((n + per - 1) / per); }
 
 // The search with its output either in host memory (out_host) or in device memory (d_out).
 int knn_gpu_impl(rbfx_ctx* ctx, int32_t n_nodes, const double* xyz, int32_t k, int32_t* out_host, int32_t* d_out,
@@ -125,77 +461,98 @@ int knn_gpu_impl(rbfx_ctx* ctx, int32_t n_nodes, const double* xyz, int32_t k, i
     RBFX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
     // host kd-tree answers for `rows`, written to the output wherever it lives
-    auto host_rows = [&](const std::vector<int32_t>& rows) -> int {
+    auto host_rows = [&](std::vector<int32_t>& rows) -> int {
         if (n_host_rows) *n_host_rows = (int32_t)rows.size();
         if (rows.empty()) return RBFX_OK;
         if (out_host) return rbfx_knn_kdtree_rows(n_nodes, xyz, k, rows.data(), (int32_t)rows.size(), out_host, 0);
-        std::vector<int32_t> tmp(rows.size() * (size_t)k);
-        int rc = rbfx_knn_kdtree_rows(n_nodes, xyz, k, rows.data(), (int32_t)rows.size(), tmp.data(), 1);
+        const size_t m = rows.size();
+        rows.resize(m * ((size_t)k + 1));  // the rows, then their lists
+        int rc = rbfx_knn_kdtree_rows(n_nodes, xyz, k, rows.data(), (int32_t)m, rows.data() + m, 1);
         if (rc != RBFX_OK) return rc;
-        for (size_t r = 0; r < rows.size(); r++)
-            RBFX_HIP_CHECK(ctx, hipMemcpyAsync(d_out + (size_t)rows[r] * k, tmp.data() + r * k, sizeof(int32_t) * k,
-                                               hipMemcpyHostToDevice, st));
+        DevBuf put;
+        if (hipMalloc(&put.p, rows.size() * sizeof(int32_t)) != hipSuccess)
+            return rbfx_fail(ctx, RBFX_E_NOMEM, "knn_gpu: rows from the host");
+        RBFX_HIP_CHECK(ctx, hipMemcpyAsync(put.p, rows.data(), rows.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
+        knn_put_rows_kernel<<<blocks_for(m * k, 256), 256, 0, st>>>((int32_t*)put.p, (int32_t*)put.p + m, (int)m, k, d_out);
+        RBFX_LAUNCH_CHECK(ctx, "knn_put_rows_kernel");
         RBFX_HIP_CHECK(ctx, hipStreamSynchronize(st));
         return RBFX_OK;
     };
-    // the GPU list holds k+1 entries per query in LDS (64 or 32 queries per block)
-    const int B = (size_t)(k + 1) * 64 * 12 <= 65536 ? 64 : 32;
-    if (k + 1 > n_nodes || (size_t)(k + 1) * B * 12 > 65536) {
+    if (k + 1 > n_nodes || k + 1 > KNN_MAX_K1) {
         for (size_t i = 0; i < 3 * (size_t)n_nodes; i++)
             if (!std::isfinite(xyz[i])) return rbfx_fail(ctx, RBFX_E_INVALID, "knn_gpu: non-finite coordinate");
         std::vector<int32_t> rows((size_t)n_nodes);
         for (int32_t i = 0; i < n_nodes; i++) rows[(size_t)i] = i;
         return host_rows(rows);
     }
-    double lo[3], h = 1.0;
-    int32_t g[3];
-    std::vector<int32_t> cstart, pid;
-    std::vector<double> pts;
-    if (rbfx_knn_grid_bin(n_nodes, xyz, k, lo, &h, g, cstart, pts, pid) != RBFX_OK)
-        return rbfx_fail(ctx, RBFX_E_INVALID, "knn_gpu: non-finite coordinate");
-    const size_t n_cells = (size_t)g[0] * g[1] * g[2];
-    DevBufs db;
-    const size_t sz[6] = {sizeof(double) * 3 * (size_t)n_nodes, sizeof(int32_t) * (size_t)n_nodes,
-                          sizeof(int32_t) * (n_cells + 1), sizeof(double) * 3 * (size_t)n_nodes,
-                          d_out ? 0 : sizeof(int32_t) * (size_t)n_nodes * k, sizeof(int32_t) * (size_t)n_nodes};
-    for (int b = 0; b < 6; b++) {
-        if (!sz[b]) continue;
-        hipError_t e = hipMalloc(&db.p[b], sz[b]);
-        if (e != hipSuccess) return rbfx_fail(ctx, RBFX_E_NOMEM, "knn_gpu: %s", hipGetErrorString(e));
-    }
-    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(db.p[0], pts.data(), sz[0], hipMemcpyHostToDevice, st));
-    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(db.p[1], pid.data(), sz[1], hipMemcpyHostToDevice, st));
-    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(db.p[2], cstart.data(), sz[2], hipMemcpyHostToDevice, st));
-    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(db.p[3], xyz, sz[3], hipMemcpyHostToDevice, st));
+    const size_t n = (size_t)n_nodes;
+    const int max_cells = (int)std::min<size_t>((size_t)1 << 24, std::max<size_t>(4096, 16 * n));
+    double *d_xyz = nullptr, *part = nullptr;
+    Plan* plan = nullptr;
+    Point* pts = nullptr;
+    uint8_t* seen = nullptr;
+    int *count = nullptr, *start = nullptr, *total = nullptr;
+    int32_t *ties = nullptr, *out = d_out;
+    auto carve = [&](Carver& m) {
+        m.take(&d_xyz, 3 * n);
+        m.take(&pts, n);
+        m.take(&part, BOUND_BLOCKS * 7);
+        m.take(&plan, 1);
+        m.take(&seen, (size_t)max_cells);
+        m.take(&count, (size_t)max_cells);
+        m.take(&start, (size_t)max_cells + 1);
+        m.take(&total, (size_t)max_cells / SCAN_TILE + 1);
+        m.take(&ties, n);
+        if (out_host) m.take(&out, n * k);
+    };
+    Carver m;
+    carve(m);
+    DevBuf mem;
+    hipError_t e = hipMalloc(&mem.p, m.used);
+    if (e != hipSuccess) return rbfx_fail(ctx, RBFX_E_NOMEM, "knn_gpu: %s", hipGetErrorString(e));
+    m = Carver{(unsigned char*)mem.p};
+    carve(m);
+    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(d_xyz, xyz, 3 * n * sizeof(double), hipMemcpyHostToDevice, st));
+    RBFX_HIP_CHECK(ctx, hipMemsetAsync(seen, 0, (size_t)max_cells, st));
+    const int bound_blocks = (int)std::min<size_t>(BOUND_BLOCKS, (n + 255) / 256);
+    knn_bounds_kernel<<<bound_blocks, 256, 0, st>>>(d_xyz, n_nodes, part);
+    knn_levels_kernel<<<1, 64, 0, st>>>(part, bound_blocks, max_cells, plan);
+    knn_mark_kernel<<<blocks_for(n, 256), 256, 0, st>>>(d_xyz, n_nodes, plan, seen);
+    knn_occupied_kernel<<<dim3(32, KNN_LEVELS), 256, 0, st>>>(plan, seen);
+    knn_choose_kernel<<<1, 64, 0, st>>>(plan, n_nodes, k, max_cells);
+    RBFX_LAUNCH_CHECK(ctx, "knn grid kernels");
+    Plan host;
+    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(&host, plan, sizeof(Plan), hipMemcpyDeviceToHost, st));
+    RBFX_HIP_CHECK(ctx, hipStreamSynchronize(st));
+    if (host.bad) return rbfx_fail(ctx, RBFX_E_INVALID, "knn_gpu: non-finite coordinate");
+    const int n_cells = host.grid.n_cells, tiles = (int)blocks_for(n_cells, SCAN_TILE);
+    RBFX_HIP_CHECK(ctx, hipMemsetAsync(count, 0, (size_t)n_cells * sizeof(int), st));
+    knn_count_kernel<<<blocks_for(n, 256), 256, 0, st>>>(d_xyz, n_nodes, plan, count);
+    knn_scan_kernel<<<tiles, SCAN_THREADS, 0, st>>>(count, n_cells, start, total);
+    knn_scan_totals_kernel<<<1, 1024, 0, st>>>(total, tiles);
+    knn_scan_add_kernel<<<blocks_for((size_t)n_cells + 1, 256), 256, 0, st>>>(start, n_cells, total, n_nodes);
+    knn_scatter_kernel<<<blocks_for(n, 256), 256, 0, st>>>(d_xyz, n_nodes, plan, start, count, pts);
     KnnArgs a;
-    a.pts = (const double*)db.p[0];
-    a.pid = (const int32_t*)db.p[1];
-    a.cstart = (const int32_t*)db.p[2];
-    a.q = (const double*)db.p[3];
-    a.out = d_out ? d_out : (int32_t*)db.p[4];
-    a.flag = (int32_t*)db.p[5];
+    a.pts = pts;
+    a.start = start;
+    a.plan = plan;
+    a.out = out;
+    a.ties = ties;
     a.n = n_nodes;
     a.k = k;
-    a.gx = g[0];
-    a.gy = g[1];
-    a.gz = g[2];
-    a.lo0 = lo[0];
-    a.lo1 = lo[1];
-    a.lo2 = lo[2];
-    a.inv_h = 1.0 / h;
-    a.h = h;
-    const size_t lds = (size_t)(k + 1) * B * 12;
-    knn_grid_kernel<<<(n_nodes + B - 1) / B, B, lds, st>>>(a);
+    a.nb = (int)((blocks_for(n, KNN_WAVES * KNN_PER_WAVE) + 7) / 8 * 8);
+    knn_grid_kernel<<<a.nb, 64 * KNN_WAVES, 0, st>>>(a);
     RBFX_LAUNCH_CHECK(ctx, "knn_grid_kernel");
-    std::vector<int32_t> flag((size_t)n_nodes);
     if (out_host)
-        RBFX_HIP_CHECK(ctx, hipMemcpyAsync(out_host, db.p[4], sizeof(int32_t) * (size_t)n_nodes * k,
-                                           hipMemcpyDeviceToHost, st));
-    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(flag.data(), db.p[5], sz[5], hipMemcpyDeviceToHost, st));
+        RBFX_HIP_CHECK(ctx, hipMemcpyAsync(out_host, out, sizeof(int32_t) * n * k, hipMemcpyDeviceToHost, st));
+    int n_ties = 0;
+    RBFX_HIP_CHECK(ctx, hipMemcpyAsync(&n_ties, &plan->n_ties, sizeof(int), hipMemcpyDeviceToHost, st));
     RBFX_HIP_CHECK(ctx, hipStreamSynchronize(st));
-    std::vector<int32_t> rows;
-    for (int32_t i = 0; i < n_nodes; i++)
-        if (flag[(size_t)i]) rows.push_back(i);
+    std::vector<int32_t> rows((size_t)n_ties);
+    if (n_ties) {
+        RBFX_HIP_CHECK(ctx, hipMemcpyAsync(rows.data(), ties, (size_t)n_ties * sizeof(int32_t), hipMemcpyDeviceToHost, st));
+        RBFX_HIP_CHECK(ctx, hipStreamSynchronize(st));
+    }
     return host_rows(rows);
 }
 
@@ -217,7 +574,7 @@ int rbfx_knn_gpu(rbfx_ctx* ctx, int32_t n_nodes, const double* xyz, int32_t k, i
 
 // The same lists written to device memory (d_out_idx: n_nodes * k int32 on the context's
 // device), so that the weights and operators can be built from them without a round trip
-// through host memory. Tie rows are recomputed on the host and uploaded row by row.
+// through host memory. Tie rows are recomputed on the host and uploaded.
 int rbfx_knn_gpu_device(rbfx_ctx* ctx, int32_t n_nodes, const double* xyz, int32_t k, int32_t* d_out_idx,
                         int32_t* n_host_rows) {
     if (!ctx) return RBFX_E_INVALID;

@@ -646,17 +646,6 @@ void stokes_free(rbfx_stokes* S) {
         if (p) hipFree(p);
 }
 
-// Pieces of one allocation, each on 256 bytes: carve once without memory for the size, then with it.
-struct Carver {
-    unsigned char* base = nullptr;
-    size_t used = 0;
-    template <typename T>
-    void take(T** p, size_t n) {
-        if (base) *p = reinterpret_cast<T*>(base + used);
-        used += (n * sizeof(T) + 255) / 256 * 256;
-    }
-};
-
 // One sweep's order on the host: rows level by level, each row's task and chunk, and the chunks
 // (up to SWEEP_ROWS rows of a level) with the place of their packed entries.
 struct HostSide {
