@@ -232,6 +232,18 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu((sizeo
     }
 }
 
+// One field, four lanes per row (share 6); lane o of a quad writes operator o's derivative.
+template <typename WT, typename UT, typename AT, int NOPS>
+__global__ void __launch_bounds__(64) ell_spmm_quad_kernel(const int32_t* __restrict__ idx_t, const WT* __restrict__ w_t,
+                                                           const UT* __restrict__ u, UT* __restrict__ out,
+                                                           const int32_t* __restrict__ order, int n_rows, int width, int nb) {
+    const int p = xcd_tile(blockIdx.x, nb) * 16 + (int)threadIdx.x / 4, q = threadIdx.x % 4;
+    if (p >= n_rows) return;  // whole quads
+    const int row = ell_row_at(order, p);
+    const AT d = ell_gather_dot_quad<WT, UT, AT, NOPS>(idx_t, w_t, u, p, width, q);
+    if (q < NOPS) out[(size_t)q * n_rows + row] = (UT)d;
+}
+
 // Single operator `op` out of an interleaved set of n_ops (one field).
 template <typename WT, typename UT, typename AT>
 __global__ void __launch_bounds__(256) ell_spmv_strided_kernel(const int32_t* __restrict__ idx_t,
@@ -335,6 +347,13 @@ int launch_spmm_lds(rbfx_ell* e, const EllTune& t, int F, const void* u, void* o
 template <typename WT, typename UT, typename AT, int NOPS>
 int launch_spmm_fpt(rbfx_ell* e, const EllTune& t, int F, const void* u, void* out) {
     if (t.share == 4 || t.share == 5) return launch_spmm_lds<WT, UT, AT, NOPS>(e, t, F, u, out);
+    if (t.share == 6) {
+        const int nb = grid_blocks((e->n_rows + 15) / 16);
+        ell_spmm_quad_kernel<WT, UT, AT, NOPS><<<nb, 64, 0, e->ctx->stream>>>(e->idx_t, (const WT*)e->w_t, (const UT*)u, (UT*)out,
+                                                                             e->order, e->n_rows, e->width, nb);
+        RBFX_LAUNCH_CHECK(e->ctx, "ell_spmm_quad_kernel");
+        return RBFX_OK;
+    }
     const int fpt = t.fpt, block = t.block;
     int G = F / fpt;
     int R = block / G;

@@ -684,6 +684,50 @@ __device__ __forceinline__ void ell_gather_dot_lds_mfma(const uint16_t* __restri
     g.finish(lds, fofs, acc);
 }
 
+// One field on four lanes per row (share 6), for operator sets too small to fill the chip with a
+// row per lane. Lane q of the quad gathers slots q, q + 4, ... and multiplies for operator q
+// (lanes past the last operator repeat operator 0): it loads its operator's weight of every slot,
+// the field values are broadcast inside the quad with DPP. A chunk of 32 slots is requested at once,
+// indices and weights of the next chunk before the current one is consumed, so a stencil of up to
+// 32 nodes waits for two loads, its indices and its values. Returns operator q's sum, slots in the
+// order and with the multiply-adds of ell_gather_dot: bit-identical.
+template <typename WT, typename UT, typename AT, int NOPS>
+__device__ __forceinline__ AT ell_gather_dot_quad(const int32_t* __restrict__ idx_t, const WT* __restrict__ w_t,
+                                                  const UT* __restrict__ u, int row, int width, int q) {
+    constexpr int C = 32;
+    const size_t base = ell_row_base(row, width);
+    const int32_t* ip = idx_t + base;
+    const WT* wp = w_t + base * NOPS + (q < NOPS ? q : 0);
+    const size_t wstride = (size_t)ELL_TILE * NOPS;
+    int nb[C / 4];
+    WT w[C];
+    auto request = [&](int j0) {
+#pragma unroll
+        for (int l = 0; l < C / 4; l++)
+            if (j0 + 4 * l < width) nb[l] = ip[(size_t)min(j0 + 4 * l + q, width - 1) * ELL_TILE];
+#pragma unroll
+        for (int j = 0; j < C; j++)
+            if (j0 + j < width) w[j] = wp[(size_t)(j0 + j) * wstride];
+    };
+    AT acc = (AT)0;
+    request(0);
+    for (int j0 = 0; j0 < width; j0 += C) {
+        UT v[C / 4];
+        WT wc[C];
+#pragma unroll
+        for (int l = 0; l < C / 4; l++)
+            if (j0 + 4 * l < width) v[l] = u[nb[l]];
+#pragma unroll
+        for (int j = 0; j < C; j++) wc[j] = w[j];
+        request(j0 + C);
+        StaticFor<0, C>::run([&](auto J) {
+            constexpr int j = decltype(J)::value;
+            if (j0 + j < width) acc = fma_acc<AT>((AT)wc[j], (AT)bcast_group<4, j % 4>(v[j / 4]), acc);
+        });
+    }
+    return acc;
+}
+
 // Maps a hardware block index to a logical tile so that each of the 8 XCDs (which receive
 // blocks round-robin) works on one contiguous eighth of the rows and keeps its gathered
 // neighbourhood in its own L2.
@@ -697,7 +741,7 @@ struct EllTune {
     int fpt = 1;
     int block = 256;
     int ub = 4;     // slots per gather batch (4 or 8)
-    int share = 0;  // 1: the G = F/fpt lanes of a row split the index/weight loads (G = 2 or 4)
+    int share = 0;  // how lanes share a row's loads, as in rbfx_tune_set
 };
 
 int rbfx_ell_pick(rbfx_ell* ell, int n_fields, int field_type, int accum, int kind, EllTune* t);

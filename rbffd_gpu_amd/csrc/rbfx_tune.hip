@@ -3,11 +3,7 @@
 // A tuning table maps (kind, rows bucket, width, n_ops, fields, storage, field type,
 // accumulation) to the shape measured fastest by rbfx_tune_spmm / the autotuner in the
 // Python layer; the table lives in memory and can be saved/loaded as text so a run can reuse
-// an earlier sweep. Without an entry: an RK4 stage of an operator set with LDS staging tables
-// (rbfx_ell_build_local) that fit takes the LDS-staged shape (4 lanes per row, 16 fields,
-// batch 4; the matrix-core variant for FP32 weights, fields and accumulation); otherwise the
-// heuristic picks the largest fields-per-thread of 8/4/2/1 that divides F and keeps at most
-// 16 FP64 (32 FP32) accumulators per thread.
+// an earlier sweep. Without an entry the rules of default_shape decide.
 #include <cstdio>
 #include <map>
 #include <mutex>
@@ -48,6 +44,53 @@ bool lds_shape_fits(const rbfx_ell* e, int F, int ft, int acc, int kind, const E
     if (c.share == 5) ok = ok && c.fpt == 4 && G == 4 && e->storage != RBFX_F64 && ft == RBFX_F32 && acc == RBFX_F32;
     return ok;
 }
+
+// The shape of a set without a tuned entry. Times are of four RK4 stages, n = 31 or 50, FP64 / FP32.
+EllTune default_shape(const rbfx_ell* e, int F, int ft, int acc, int kind) {
+    const long long n = e->n_rows;
+    const bool f64 = e->storage == RBFX_F64;
+    const int cus = e->ctx->n_cu > 0 ? e->ctx->n_cu : 256;
+    // LDS-staged gathers for a set with tile tables whose records fit the LDS (60,000 rows: 80 against
+    // 106 us in FP64)
+    if (e->lt > 0 && e->n_ops >= 3 && F == 16 && e->lt * 4 <= 512) {
+        const size_t rec = (size_t)F * (ft == RBFX_F64 ? 8 : 4);
+        if ((size_t)e->k_max * rec <= (size_t)e->lds_limit)
+            return EllTune{4, e->lt * 4, 4, !f64 && ft == RBFX_F32 && acc == RBFX_F32 ? 5 : 4};
+    }
+    // One field of few rows: four lanes per row, while all waves of 16 rows are on the chip together
+    // (two per SIMD in FP64, four in FP32). 4096 / 20,000 rows: 20.0 / 21.1 us in FP64 against 21.7 / 25.0
+    // with a lane per row, 19.8 / 20.1 against 25.3 / 26.9 in FP32; at 40,000 rows 35.9 against 33.7 in
+    // FP64, at 80,000 61 against 58 in FP32. Short stencils gain nothing (n = 17: 19.4 against 18.3). A
+    // single operator's weights are loaded by all four lanes: not for long stencils (n = 101: 9.5 against
+    // 9.0 us an apply) nor beyond two waves per SIMD (60,000 rows in FP32: 8.9 against 7.6).
+    if (F == 1 && e->n_ops <= 4 && e->width >= 24 && n <= 128ll * cus * (f64 || e->n_ops == 1 ? 1 : 2) &&
+        (e->n_ops > 1 || e->width <= 64))
+        return EllTune{1, 64, 8, 6};
+    // Otherwise: as many fields per thread, up to 4, as leave a wave per SIMD, for FP32 applies one per two
+    // (16 FP64 or 32 FP32 sums at most): fewer loads of the indices and weights, fewer threads. 80,000 rows x 4
+    // fields: 106 us with 4 against 112 with 2; 4096 x 4: 22 with 1 against 46 with 4; FP32: 400,000 x 8 449 with
+    // 4 against 544 with 8, 20,000 x 8 32.5 with 2 against 36.2 with 4, but 30,000 x 8 7.1 an apply with 4, 8.0 with 2.
+    const int max_acc = acc == RBFX_F64 ? 16 : 32;
+    int fpt = 1;
+    for (int c : {4, 2})
+        if (F % c == 0 && c * e->n_ops <= max_acc && n * (F / c) >= (f64 || kind == 1 ? 256ll : 128ll) * cus) {
+            fpt = c;
+            break;
+        }
+    // 64-thread blocks spread few rows over more CUs (4096 rows: 22 against 29 us), 256-thread ones keep
+    // neighbouring rows of many on one CU (400,000 rows x 2: 563 against 565, 316 against 320).
+    int block = n * (F / fpt) < 1024ll * cus ? 64 : 256;
+    // Slots per memory round trip: 16 for a single operator on one field (111 against 120 us with 4 at a
+    // million rows), else 8 (4096 rows: 22 against 25), but 4 where 8 slots of FP64 weights leave few waves:
+    // four fields on small blocks (80,000 rows x 4: 106 against more than 112; 400,000 x 8: 788 with 8, 835 with
+    // 4), applies of several operators (100,000 rows, 2: 17.8 against 18.5; 60,000 x 4 fields, 3: 12.4 with 256-thread
+    // blocks against 14.3).
+    int ub = 8;
+    if (kind == 0 && F == 1 && e->n_ops == 1) ub = 16;
+    else if (f64 && block == 64 && (kind == 0 || fpt == 4)) ub = 4;
+    if (kind == 0 && f64 && fpt > 1) block = 256;
+    return EllTune{fpt, block, ub, 0};
+}
 }  // namespace
 
 int rbfx_ell_pick(rbfx_ell* e, int F, int ft, int acc, int kind, EllTune* t) {
@@ -68,22 +111,8 @@ int rbfx_ell_pick(rbfx_ell* e, int F, int ft, int acc, int kind, EllTune* t) {
             // otherwise: the shape of a set without (fitting) tile tables, below
         }
     }
-    if ((kind == 0 || kind == 1) && e->lt > 0 && e->n_ops >= 3 && F == 16 && e->lt * 4 <= 512) {
-        const size_t rec = (size_t)F * (ft == RBFX_F64 ? 8 : 4);
-        if ((size_t)e->k_max * rec <= (size_t)e->lds_limit) {
-            const bool mx = e->storage != RBFX_F64 && ft == RBFX_F32 && acc == RBFX_F32;
-            *t = EllTune{4, e->lt * 4, 4, mx ? 5 : 4};
-            return RBFX_OK;
-        }
-    }
-    int max_acc = (acc == RBFX_F64) ? 16 : 32;
-    int fpt = 1;
-    for (int c : {8, 4, 2}) {
-        if (F % c == 0 && c * e->n_ops <= max_acc) { fpt = c; break; }
-    }
-    t->fpt = fpt;
-    t->block = 256;
-    if (!valid(F, t->fpt, t->block))
+    *t = default_shape(e, F, ft, acc, kind);
+    if (!valid(F, t->fpt, t->block) && t->share != 4 && t->share != 5)
         return rbfx_fail(e->ctx, RBFX_E_TOO_LARGE, "no launch shape for %d fields (at most 256*8)", F);
     return RBFX_OK;
 }
@@ -109,6 +138,13 @@ int rbfx_tune_set(rbfx_ell* e, int32_t kind, int32_t n_fields, int32_t field_typ
                              n_fields, fpt, batch, e->lt, e->k_max);
         std::lock_guard<std::mutex> lk(g_mu);
         g_table[make_key(e, n_fields, field_type, accum, kind)] = EllTune{fpt, e->lt * G, batch, share};
+        return RBFX_OK;
+    }
+    if (share == 6) {  // one field on four lanes per row, 64-thread blocks
+        if ((kind != 0 && kind != 1) || n_fields != 1 || fpt != 1 || block != 64 || batch != 8 || e->n_ops > 4)
+            return rbfx_fail(e->ctx, RBFX_E_INVALID, "tune_set: share 6 takes one field, fpt 1, block 64, batch 8 and at most 4 operators");
+        std::lock_guard<std::mutex> lk(g_mu);
+        g_table[make_key(e, n_fields, field_type, accum, kind)] = EllTune{1, 64, 8, 6};
         return RBFX_OK;
     }
     // batch 16: the SpMV/SpMM kernel with one field per thread only

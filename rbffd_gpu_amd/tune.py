@@ -36,6 +36,8 @@ def candidates(n_fields, kind=KIND_SPMM, n_ops=1, local=None, field_bytes=8, fp3
                     yield fpt, local[0] * G, batch, 4
                     if fp32_accum and field_bytes == 4 and fpt == 4:
                         yield fpt, local[0] * G, batch, 5
+    if n_fields == 1 and n_ops <= 4:
+        yield 1, 64, 8, 6  # four lanes per row
     for fpt in (1, 2, 4, 8):
         if n_fields % fpt:
             continue
