@@ -25,7 +25,7 @@
 #include <type_traits>
 #include <vector>
 
-#include "rbfx_internal.h"
+#include "rbfx_ell_common.h"
 
 namespace {
 
@@ -647,7 +647,10 @@ __device__ __forceinline__ unsigned wave_umax32_uniform(unsigned v) {
 __device__ __forceinline__ unsigned long long wave_umax_uniform(unsigned long long v) {
     const unsigned hi = (unsigned)(v >> 32), lo = (unsigned)v;
     const unsigned mh = wave_umax32_uniform(hi);
-    const unsigned ml = wave_umax32_uniform(hi == mh ? lo : 0u);
+    const unsigned long long at = __ballot(hi == mh);
+    // mostly one lane holds the largest high word: its low word needs no second chain
+    const unsigned ml = (at & (at - 1)) == 0 ? (unsigned)__builtin_amdgcn_readlane((int)lo, __ffsll(at) - 1)
+                                             : wave_umax32_uniform(hi == mh ? lo : 0u);
     return ((unsigned long long)mh << 32) | ml;
 }
 
@@ -1109,15 +1112,10 @@ __host__ __device__ inline int lu_pick(int m, int T) {
     return -1;
 }
 
-// Right-hand sides per wave in one back-substitution pass: LU_QC, or LU_QA when the
-// right-hand-side buffer shares R0 with the packed U (see lu_rhs_in_r0).
-constexpr int LU_QC = 4;
-__host__ __device__ constexpr int lu_qa(int W) { return W == 1 ? 4 : W == 2 ? 2 : 1; }
-
-// The right-hand-side buffer BS lives inside R0 (after the staged coordinates) when one
-// back-substitution pass of LU_QA right-hand sides per wave covers all T: the waves then read
-// their right-hand sides into registers before the packed U is written over them.
-__host__ __device__ inline bool lu_rhs_in_r0(int W, int T) { return T <= W * lu_qa(W); }
+// The right-hand-side buffer BS lives inside R0 (after the staged coordinates) when one wave
+// solves all T right-hand sides (four at a time): it reads them into registers before the packed U
+// is written over them.
+__host__ __device__ inline bool lu_rhs_in_r0(int T) { return T <= 4; }
 
 // LDS of one team, in doubles: [R0][BS: m T, unless inside R0][dg: m][amax: 8][umax: 8], then
 // [flag: 4 int] and 16-bit row numbers [perm: m][pos: 16 RT]. R0 holds the staged coordinates
@@ -1129,13 +1127,13 @@ __host__ __device__ inline bool lu_rhs_in_r0(int W, int T) { return T <= W * lu_
 // largest degree-2 system (m = 111, 4 right-hand sides) takes 50.4 KB: three workgroups fit in
 // the 160 KB of a CU (a workgroup's LDS is allocated in 2 KB steps).
 __host__ __device__ inline size_t lu_r0(int W, int RT, int NCT, int m, int n, int T) {
-    const size_t a = (size_t)5 * n + (lu_rhs_in_r0(W, T) ? (size_t)m * T : 0),
+    const size_t a = (size_t)5 * n + (lu_rhs_in_r0(T) ? (size_t)m * T : 0),
                  b = (size_t)24 * (16 * RT + 4) + (size_t)8 * (16 * W * NCT + 4), c = (size_t)m * (m - 1) / 2;
     const size_t ab = a > b ? a : b;
     return ab > c ? ab : c;
 }
 __host__ __device__ inline size_t lu_team_bytes(int W, int RT, int NCT, int m, int n, int T) {
-    const size_t d = lu_r0(W, RT, NCT, m, n, T) + (lu_rhs_in_r0(W, T) ? 0 : (size_t)m * T) + m + 16;
+    const size_t d = lu_r0(W, RT, NCT, m, n, T) + (lu_rhs_in_r0(T) ? 0 : (size_t)m * T) + m + 16;
     const size_t i = 4 * sizeof(int) + ((size_t)m + 16 * RT) * sizeof(short);
     return (d * sizeof(double) + i + 15) / 16 * 16;
 }
@@ -1146,6 +1144,16 @@ __host__ __device__ inline size_t lu_team_bytes(int W, int RT, int NCT, int m, i
 __device__ __forceinline__ int opaque_v(int x) {
     asm volatile("" : "+v"(x));
     return x;
+}
+
+// The value of lane 16 r + K in every lane of row r (16 lanes).
+template <int K>
+__device__ __forceinline__ double row_bcast(double v) {
+    constexpr int ctrl = 0x150 + K;  // DPP row_newbcast:K
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, ctrl, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), ctrl, 0xF, 0xF, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
 template <int W>
@@ -1211,7 +1219,7 @@ __device__ __attribute__((noinline)) void lu_team(const WParams& P, int start, i
     S.perm = nullptr;
     // team LDS
     unsigned char* base = smem + (size_t)team * lu_team_bytes(W, RT, NCT, m, n, T);
-    const bool rhs_in_r0 = lu_rhs_in_r0(W, T);
+    const bool rhs_in_r0 = lu_rhs_in_r0(T);
     double* R0 = (double*)base;
     double* BS = rhs_in_r0 ? R0 + 5 * n : R0 + lu_r0(W, RT, NCT, m, n, T);
     double* dg = R0 + lu_r0(W, RT, NCT, m, n, T) + (rhs_in_r0 ? 0 : (size_t)m * T);
@@ -1283,6 +1291,9 @@ __device__ __attribute__((noinline)) void lu_team(const WParams& P, int start, i
         const int ctp = kp >> 4, owner = ctp % W, slot = ctp / W, gp = (kp & 15) >> 2;
         double* Lb = Lbuf + ((kp / KB) & 1) * (KB * PS);
         if (wt == owner) {
+            // the team waits for this wave at the next barrier: it issues ahead of the waves of the other
+            // workgroups on its SIMD (101 nodes: 9.59 -> 9.41 ms per 40,000 stencils)
+            if (W > 1) __builtin_amdgcn_s_setprio(3);
             // panel column kp + j sits in register gp + j/4 of lane group j%4
 #pragma unroll
             for (int sl = 0; sl < NCT; sl++)
@@ -1387,6 +1398,7 @@ __device__ __attribute__((noinline)) void lu_team(const WParams& P, int start, i
                         }
                 }
         }
+        if (W > 1) __builtin_amdgcn_s_setprio(0);
         team_sync<W>();  // multipliers, pivots and pos of this panel are visible
         const int kdone = kp + npn;  // columns < kdone are finished
         // 1. the pivot rows' values on this wave's live tiles: every lane checks whether its
@@ -1505,108 +1517,78 @@ __device__ __attribute__((noinline)) void lu_team(const WParams& P, int start, i
         }
         return um;
     };
-    // Back substitution of the right-hand sides t = t0 + wt + W q, q < Q: b[q][h] holds
-    // unknown lane + 64 h (pivot order); then the weights out.
-    auto load_rhs = [&](auto qtag, auto& b, int t0) {
-        constexpr int Q = decltype(qtag)::value;
+    // Back substitution of four right-hand sides in one wave: lane 16 q + i holds unknowns i, i + 16, ...
+    // (pivot order) of right-hand side t0 + q, so one division and one broadcast inside each row of 16
+    // lanes serve all four. Every unknown sees the operations of the one-wave kernels in their order.
+    // It is a chain of m divisions (about 80 cycles each) with one broadcast and one product between
+    // them: the unrolled steps put U's loads, whose addresses depend on nothing, ahead of the chain, and
+    // one wave per stencil leaves the SIMDs to the other workgroups. A loop over the unknowns with one
+    // right-hand side per wave (its pivot element read by lane number, each wave dividing for itself)
+    // took 79,000 cycles of an m = 111 stencil, this takes 33,000: 40,000 stencils of 101 nodes
+    // 10.3 -> 9.4 ms, of 31 nodes 1.94 -> 1.70 ms, with the priorities and the shorter pivot search.
+    // The loads of rows past k stay inside the team's LDS (the diagonal and the maxima follow the packed
+    // U: 15 doubles at most are read past it) and their products are not kept.
+    const int li = lane & 15, lq = lane >> 4;
+    auto load_rhs = [&](double (&b)[RT], int t0) {
 #pragma unroll
-        for (int h = 0; h < RR; h++) {
-            const int i = lane + WAVE * h;
-#pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const int t = t0 + wt + W * q;
-                b[q][h] = (t < T && i < m) ? BS[i * T + t] : 0.0;
-            }
-        }
+        for (int h = 0; h < RT; h++) b[h] = (t0 + lq < T && 16 * h + li < m) ? BS[(16 * h + li) * T + t0 + lq] : 0.0;
     };
-    auto back_sub = [&](auto qtag, auto& b, int t0) {
-        constexpr int Q = decltype(qtag)::value;
-        // column k of U (rows < k) and the pivot u_kk are loaded one step ahead
-        double ucn[RR], ukn = dg[m - 1];
+    auto back_sub = [&](double (&b)[RT], int t0) {
+        __builtin_amdgcn_s_setprio(3);  // the team's other waves have nothing left to do
+        StaticFor<0, 16 * RT>::run([&](auto KR) {
+            constexpr int k = 16 * RT - 1 - decltype(KR)::value, h = k / 16, kk = k % 16;
+            if (k < m) {
+                const double* uc = Upk + k * (k - 1) / 2 + li;  // column k of U, rows < k
+                double u[h + 1];
 #pragma unroll
-        for (int h = 0; h < RR; h++)
-            ucn[h] = (lane + WAVE * h < m - 1) ? Upk[(size_t)(m - 1) * (m - 2) / 2 + lane + WAVE * h] : 0.0;
-        for (int k = m - 1; k >= 0; k--) {
-            double ucol[RR];
+                for (int g = 0; g <= h; g++) u[g] = uc[16 * g];
+                const double x = row_bcast<kk>(b[h]) / dg[k];
 #pragma unroll
-            for (int h = 0; h < RR; h++) ucol[h] = ucn[h];
-            const double ukk = ukn;
-            if (k > 0) {
-                const double* uc = Upk + (size_t)(k - 1) * (k - 2) / 2;
-#pragma unroll
-                for (int h = 0; h < RR; h++) ucn[h] = (lane + WAVE * h < k - 1) ? uc[lane + WAVE * h] : 0.0;
-                ukn = dg[k - 1];
+                for (int g = 0; g < h; g++) b[g] -= u[g] * x;
+                b[h] = li < kk ? b[h] - u[h] * x : li == kk ? x : b[h];
             }
-#pragma unroll
-            for (int q = 0; q < Q; q++) {
-                if (t0 + wt + W * q >= T) continue;
-                const double bk = readlane_f64((RR == 1 || k < WAVE) ? b[q][0] : b[q][RR - 1], k & (WAVE - 1));
-                const double x = bk / ukk;
-#pragma unroll
-                for (int h = 0; h < RR; h++) {
-                    const int i = lane + WAVE * h;
-                    if (i < k)
-                        b[q][h] -= ucol[h] * x;
-                    else if (i == k)
-                        b[q][h] = x;
-                }
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int q = 0; q < Q; q++) {
-            const int t = t0 + wt + W * q;
-            if (t >= T) continue;
+        });
+        __builtin_amdgcn_s_setprio(0);
+        const int t = t0 + lq;
+        if (t < T && writer) {
             const double scale = (P.types[t] == RBFX_HV) ? P.hv_scale : 1.0;
 #pragma unroll
-            for (int h = 0; h < RR; h++) {
-                const int i = lane + WAVE * h;
-                if (i < n && writer) P.w[(size_t)t * P.nnz + S.off + i] = b[q][h] * scale;
-            }
+            for (int h = 0; h < RT; h++)
+                if (16 * h + li < n) P.w[(size_t)t * P.nnz + S.off + 16 * h + li] = b[h] * scale;
         }
     };
     // x by unknown into BS, for the diagnostics
-    auto keep_x = [&](auto qtag, auto& b, int t0) {
-        constexpr int Q = decltype(qtag)::value;
+    auto keep_x = [&](double (&b)[RT], int t0) {
 #pragma unroll
-        for (int q = 0; q < Q; q++) {
-            const int t = t0 + wt + W * q;
-            if (t >= T) continue;
-#pragma unroll
-            for (int h = 0; h < RR; h++) {
-                const int i = lane + WAVE * h;
-                if (i < m) BS[i * T + t] = b[q][h];
-            }
-        }
+        for (int h = 0; h < RT; h++)
+            if (t0 + lq < T && 16 * h + li < m) BS[(16 * h + li) * T + t0 + lq] = b[h];
     };
     lane = opaque_v(lane);
     tt = wt * WAVE + lane;
-    if (rhs_in_r0) {
-        using QA = std::integral_constant<int, lu_qa(W)>;
+    if (rhs_in_r0) {  // at most four right-hand sides: wave 0 solves them
         store_rows(false, true);
         team_sync<W>();
-        double b[QA::value][RR];
-        load_rhs(QA{}, b, 0);
-        team_sync<W>();  // every wave holds its right-hand sides: BS may be overwritten
+        double b[RT];
+        if (wt == 0) load_rhs(b, 0);
+        team_sync<W>();  // wave 0 holds the right-hand sides: BS may be overwritten
         const double um = wave_max(store_rows(true, false));
         if (lane == 0) umaxw[wt] = um;
         team_sync<W>();
-        back_sub(QA{}, b, 0);
+        if (wt == 0) back_sub(b, 0);
         if (diag) {
-            team_sync<W>();  // every wave has read the packed U under BS
-            keep_x(QA{}, b, 0);
+            team_sync<W>();  // wave 0 has read the packed U under BS
+            if (wt == 0) keep_x(b, 0);
         }
     } else {
-        using QC = std::integral_constant<int, LU_QC>;
         const double um = wave_max(store_rows(true, true));
         if (lane == 0) umaxw[wt] = um;
         team_sync<W>();
-        for (int t0 = 0; t0 < T; t0 += W * LU_QC) {
-            double b[LU_QC][RR];
-            load_rhs(QC{}, b, t0);
-            back_sub(QC{}, b, t0);
+        for (int t0 = 4 * wt; t0 < T; t0 += 4 * W) {
+            double b[RT];
+            load_rhs(b, t0);
+            back_sub(b, t0);
             // each wave overwrites only the columns of BS it has read itself
-            if (diag) keep_x(QC{}, b, t0);
+            if (diag) keep_x(b, t0);
         }
     }
     if (tt == 0 && writer) P.fail_flags[s] = 0;
