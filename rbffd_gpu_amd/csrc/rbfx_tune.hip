@@ -80,6 +80,11 @@ EllTune default_shape(const rbfx_ell* e, int F, int ft, int acc, int kind) {
     // 64-thread blocks spread few rows over more CUs (4096 rows: 22 against 29 us), 256-thread ones keep
     // neighbouring rows of many on one CU (400,000 rows x 2: 563 against 565, 316 against 320).
     int block = n * (F / fpt) < 1024ll * cus ? 64 : 256;
+    // A row's fields stay in one block: rows of more lanes than it has take 256-thread blocks, and beyond
+    // 256 lanes the most fields per thread, so that every field count up to 256 * 8 that divides finds a shape.
+    if (F / fpt > block) block = 256;
+    for (int c : {8, 4, 2})
+        if (F / fpt > block && F % c == 0 && c * e->n_ops <= max_acc) fpt = c;
     // Slots per memory round trip: 16 for a single operator on one field (111 against 120 us with 4 at a
     // million rows), else 8 (4096 rows: 22 against 25), but 4 where 8 slots of FP64 weights leave few waves:
     // four fields on small blocks (80,000 rows x 4: 106 against more than 112; 400,000 x 8: 788 with 8, 835 with
@@ -87,7 +92,7 @@ EllTune default_shape(const rbfx_ell* e, int F, int ft, int acc, int kind) {
     // blocks against 14.3).
     int ub = 8;
     if (kind == 0 && F == 1 && e->n_ops == 1) ub = 16;
-    else if (f64 && block == 64 && (kind == 0 || fpt == 4)) ub = 4;
+    else if (fpt == 8 || (f64 && block == 64 && (kind == 0 || fpt == 4))) ub = 4;
     if (kind == 0 && f64 && fpt > 1) block = 256;
     return EllTune{fpt, block, ub, 0};
 }
