@@ -434,10 +434,10 @@ int rbfx_ell_create(rbfx_ctx* ctx, int32_t n_rows, int32_t n_cols, int32_t width
     size_t wbytes = slots * n_ops * (storage == RBFX_F64 ? sizeof(double) : sizeof(float));
     int* d_bad = nullptr;
     hipError_t err;
-    if ((err = hipMalloc(&e->idx_t, slots * sizeof(int32_t))) != hipSuccess || (err = hipMalloc(&e->w_t, wbytes)) != hipSuccess ||
-        (err = hipMalloc(&d_bad, sizeof(int))) != hipSuccess) {
-        hipFree(e->idx_t);
-        hipFree(e->w_t);
+    if ((err = rbfx_pool_alloc(ctx, &e->idx_t, slots * sizeof(int32_t))) != hipSuccess || (err = rbfx_pool_alloc(ctx, &e->w_t, wbytes)) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &d_bad, sizeof(int))) != hipSuccess) {
+        rbfx_pool_free(ctx, e->idx_t);
+        rbfx_pool_free(ctx, e->w_t);
         delete e;
         return rbfx_fail(ctx, RBFX_E_NOMEM, "ell_create: allocation failed: %s", hipGetErrorString(err));
     }
@@ -448,7 +448,7 @@ int rbfx_ell_create(rbfx_ctx* ctx, int32_t n_rows, int32_t n_cols, int32_t width
     ell_validate_kernel<<<(unsigned)((total_in + 255) / 256), 256, 0, ctx->stream>>>(d_idx, total_in, n_cols, d_bad);
     hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, ctx->stream);
     err = hipStreamSynchronize(ctx->stream);
-    hipFree(d_bad);
+    rbfx_pool_free(ctx, d_bad);
     if (err != hipSuccess || bad) {
         int code = err != hipSuccess ? RBFX_E_HIP : RBFX_E_INVALID;
         rbfx_ell_destroy(e);
@@ -482,10 +482,10 @@ int rbfx_ell_create(rbfx_ctx* ctx, int32_t n_rows, int32_t n_cols, int32_t width
 }
 
 static void free_local(rbfx_ell* e) {
-    hipFree(e->loc_pos);
-    hipFree(e->loc_off);
-    hipFree(e->loc_nodes);
-    hipFree(e->loc_idx);
+    rbfx_pool_free(e->ctx, e->loc_pos);
+    rbfx_pool_free(e->ctx, e->loc_off);
+    rbfx_pool_free(e->ctx, e->loc_nodes);
+    rbfx_pool_free(e->ctx, e->loc_idx);
     e->loc_pos = e->loc_off = e->loc_nodes = nullptr;
     e->loc_idx = nullptr;
     e->lt = e->k_max = e->n_ltiles = 0;
@@ -495,9 +495,9 @@ void rbfx_ell_destroy(rbfx_ell* e) {
     if (!e) return;
     hipSetDevice(e->ctx->device);
     hipStreamSynchronize(e->ctx->stream);
-    hipFree(e->idx_t);
-    hipFree(e->w_t);
-    hipFree(e->order);
+    rbfx_pool_free(e->ctx, e->idx_t);
+    rbfx_pool_free(e->ctx, e->w_t);
+    rbfx_pool_free(e->ctx, e->order);
     free_local(e);
     delete e;
 }
@@ -519,15 +519,15 @@ static int local_tables_host(rbfx_ell* e, int tile_rows, int max_nodes, LocalTab
     uint16_t* d_lidx = nullptr;
     hipError_t err;
     auto drop = [&]() {
-        hipFree(d_pos);
-        hipFree(d_off);
-        hipFree(d_nodes);
-        hipFree(d_lidx);
+        rbfx_pool_free(ctx, d_pos);
+        rbfx_pool_free(ctx, d_off);
+        rbfx_pool_free(ctx, d_nodes);
+        rbfx_pool_free(ctx, d_lidx);
     };
-    if ((err = hipMalloc(&d_pos, pos.size() * sizeof(int32_t))) != hipSuccess ||
-        (err = hipMalloc(&d_off, off.size() * sizeof(int32_t))) != hipSuccess ||
-        (err = hipMalloc(&d_nodes, std::max<size_t>(1, nodes.size()) * sizeof(int32_t))) != hipSuccess ||
-        (err = hipMalloc(&d_lidx, lidx.size() * sizeof(uint16_t))) != hipSuccess) {
+    if ((err = rbfx_pool_alloc(ctx, &d_pos, pos.size() * sizeof(int32_t))) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &d_off, off.size() * sizeof(int32_t))) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &d_nodes, std::max<size_t>(1, nodes.size()) * sizeof(int32_t))) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &d_lidx, lidx.size() * sizeof(uint16_t))) != hipSuccess) {
         drop();
         return rbfx_fail(ctx, RBFX_E_NOMEM, "ell_build_local: %s", hipGetErrorString(err));
     }
@@ -601,13 +601,13 @@ int rbfx_ell_set_row_order(rbfx_ell* e, const int32_t* d_order) {
     hipError_t err;
     auto release = [&]() {
         hipStreamSynchronize(s);
-        hipFree(d_count);
-        hipFree(d_old_pos);
-        hipFree(d_new_order);
-        hipFree(idx_n);
-        hipFree(w_n);
+        rbfx_pool_free(ctx, d_count);
+        rbfx_pool_free(ctx, d_old_pos);
+        rbfx_pool_free(ctx, d_new_order);
+        rbfx_pool_free(ctx, idx_n);
+        rbfx_pool_free(ctx, w_n);
     };
-    if ((err = hipMalloc(&d_count, sizeof(int) * ((size_t)n + 2))) != hipSuccess) {
+    if ((err = rbfx_pool_alloc(ctx, &d_count, sizeof(int) * ((size_t)n + 2))) != hipSuccess) {
         release();
         return rbfx_fail(ctx, RBFX_E_NOMEM, "ell_set_row_order: allocation failed: %s", hipGetErrorString(err));
     }
@@ -635,10 +635,10 @@ int rbfx_ell_set_row_order(rbfx_ell* e, const int32_t* d_order) {
         e->layout_version++;
         return RBFX_OK;
     }
-    if ((err = hipMalloc(&d_old_pos, sizeof(int32_t) * (size_t)n)) != hipSuccess ||
-        (err = hipMalloc(&d_new_order, sizeof(int32_t) * (size_t)n)) != hipSuccess ||
-        (err = hipMalloc(&idx_n, sizeof(int32_t) * entries)) != hipSuccess ||
-        (err = hipMalloc(&w_n, wsz * entries * e->n_ops)) != hipSuccess) {
+    if ((err = rbfx_pool_alloc(ctx, &d_old_pos, sizeof(int32_t) * (size_t)n)) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &d_new_order, sizeof(int32_t) * (size_t)n)) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &idx_n, sizeof(int32_t) * entries)) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &w_n, wsz * entries * e->n_ops)) != hipSuccess) {
         release();
         return rbfx_fail(ctx, RBFX_E_NOMEM, "ell_set_row_order: allocation failed: %s", hipGetErrorString(err));
     }
@@ -655,14 +655,14 @@ int rbfx_ell_set_row_order(rbfx_ell* e, const int32_t* d_order) {
         release();
         return rbfx_fail(ctx, RBFX_E_HIP, "ell_set_row_order: reorder failed: %s", hipGetErrorString(err));
     }
-    hipFree(e->idx_t);
-    hipFree(e->w_t);
-    hipFree(e->order);
+    rbfx_pool_free(ctx, e->idx_t);
+    rbfx_pool_free(ctx, e->w_t);
+    rbfx_pool_free(ctx, e->order);
     e->idx_t = idx_n;
     e->w_t = w_n;
     e->order = d_new_order;
     if (flags[1] == 0) {  // the identity: node order, which the kernels take without an order array
-        hipFree(e->order);
+        rbfx_pool_free(ctx, e->order);
         e->order = nullptr;
     }
     free_local(e);  // the local tables describe the previous layout

@@ -241,17 +241,17 @@ bool rbfx_local_tables_device(rbfx_ell* e, int lt, int cap, size_t lds_limit, Lo
     const size_t ints = 2 * (size_t)n + 5 * (size_t)n_chunks;
     auto fail = [&](hipError_t err, int code) {
         hipStreamSynchronize(st);
-        hipFree(scratch);
-        hipFree(T->pos);
-        hipFree(T->off);
-        hipFree(T->nodes);
-        hipFree(T->idx);
+        rbfx_pool_free(ctx, scratch);
+        rbfx_pool_free(ctx, T->pos);
+        rbfx_pool_free(ctx, T->off);
+        rbfx_pool_free(ctx, T->nodes);
+        rbfx_pool_free(ctx, T->idx);
         *T = LocalTables();
         *rc = rbfx_fail(ctx, code, "ell_build_local: %s", hipGetErrorString(err));
         return true;
     };
     hipError_t err;
-    if ((err = hipMalloc(&scratch, ints * sizeof(int32_t))) != hipSuccess) return fail(err, RBFX_E_NOMEM);
+    if ((err = rbfx_pool_alloc(ctx, &scratch, ints * sizeof(int32_t))) != hipSuccess) return fail(err, RBFX_E_NOMEM);
     int32_t *t_pos = scratch, *t_cnt = t_pos + n, *c_info = t_cnt + n, *c_base = c_info + 3 * (size_t)n_chunks;
     local_cut_kernel<<<n_chunks, CUT_THREADS, cut_lds, st>>>(e->idx_t, n, e->width, lt, cap, chunk, Hc, t_pos, t_cnt, c_info);
     std::vector<int32_t> info(3 * (size_t)n_chunks), base(2 * (size_t)n_chunks);
@@ -273,14 +273,14 @@ bool rbfx_local_tables_device(rbfx_ell* e, int lt, int cap, size_t lds_limit, Lo
     const int P = pow2_at_least(most, 64), H = std::min(HASH_MAX, pow2_at_least(2 * most, 128));
     const size_t list_lds = (size_t)H * 6 + (size_t)P * 4;
     if (most > HASH_MAX / 2 || list_lds + 1024 > lds_limit) {
-        hipFree(scratch);
+        rbfx_pool_free(ctx, scratch);
         return false;
     }
     const size_t all = (size_t)e->n_pad * e->width;
-    if ((err = hipMalloc(&T->pos, ((size_t)tiles + 1) * sizeof(int32_t))) != hipSuccess ||
-        (err = hipMalloc(&T->off, ((size_t)tiles + 1) * sizeof(int32_t))) != hipSuccess ||
-        (err = hipMalloc(&T->nodes, (size_t)std::max<long long>(1, nodes) * sizeof(int32_t))) != hipSuccess ||
-        (err = hipMalloc(&T->idx, all * sizeof(uint16_t))) != hipSuccess)
+    if ((err = rbfx_pool_alloc(ctx, &T->pos, ((size_t)tiles + 1) * sizeof(int32_t))) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &T->off, ((size_t)tiles + 1) * sizeof(int32_t))) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &T->nodes, (size_t)std::max<long long>(1, nodes) * sizeof(int32_t))) != hipSuccess ||
+        (err = rbfx_pool_alloc(ctx, &T->idx, all * sizeof(uint16_t))) != hipSuccess)
         return fail(err, RBFX_E_NOMEM);
     if ((err = hipMemcpyAsync(c_base, base.data(), base.size() * sizeof(int32_t), hipMemcpyHostToDevice, st)) != hipSuccess)
         return fail(err, RBFX_E_HIP);
@@ -293,7 +293,7 @@ bool rbfx_local_tables_device(rbfx_ell* e, int lt, int cap, size_t lds_limit, Lo
     local_list_kernel<<<tiles, LIST_THREADS, list_lds, st>>>(e->idx_t, e->width, lt, T->pos, T->off, H, P, T->nodes, T->idx);
     if ((err = hipGetLastError()) != hipSuccess || (err = hipStreamSynchronize(st)) != hipSuccess)
         return fail(err, RBFX_E_HIP);
-    hipFree(scratch);
+    rbfx_pool_free(ctx, scratch);
     T->n_tiles = tiles;
     T->k_max = most;
     return true;

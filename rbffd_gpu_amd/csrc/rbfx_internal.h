@@ -5,7 +5,9 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "rbfx.h"
@@ -31,6 +33,16 @@ struct rbfx_ctx {
     int clock_khz = 0;
     char name[256] = {0};
     std::string err;
+    // Device memory kept for the next object (rbfx_pool_alloc): blocks not in use, oldest first, and the
+    // sizes of those handed out.
+    struct Block {
+        void* p;
+        size_t bytes;
+    };
+    std::mutex pool_mu;
+    std::vector<Block> idle;
+    std::unordered_map<void*, size_t> lent;
+    size_t idle_bytes = 0, idle_max = 0;
 };
 
 // Records a formatted message on ctx (or the global slot) and returns code.
@@ -52,6 +64,26 @@ int rbfx_fail(rbfx_ctx* ctx, int code, const char* fmt, ...);
             return rbfx_fail((ctx), RBFX_E_HIP, "launch of %s failed: %s", (what),            \
                              hipGetErrorString(e_));                                          \
     } while (0)
+
+// hipMalloc that, when memory runs out, gives the context's idle blocks back and tries again.
+hipError_t rbfx_malloc(rbfx_ctx* ctx, void** p, size_t bytes);
+
+// Device memory of objects that are built and dropped again and again (operator sets, tile tables, the
+// Stokes factor, the search's scratch). Blocks of at least 1 MiB stay with the context when they
+// are freed and serve the next request of up to their size and at least 4/5 of it; contents are
+// whatever the last user left. Everything that touches such memory is work on the context's
+// stream, so a block's next use comes after its last one without a wait. At most 1/64 of the
+// device's memory and 32 blocks are kept; they are given back with the context, or when an
+// allocation fails.
+hipError_t rbfx_pool_alloc_bytes(rbfx_ctx* ctx, void** p, size_t bytes);
+void rbfx_pool_free(rbfx_ctx* ctx, void* p);
+template <typename T>
+hipError_t rbfx_pool_alloc(rbfx_ctx* ctx, T** p, size_t bytes) {
+    void* v = nullptr;
+    const hipError_t e = rbfx_pool_alloc_bytes(ctx, &v, bytes);
+    *p = static_cast<T*>(v);
+    return e;
+}
 
 // Pieces of one allocation, each on 256 bytes: carve once without memory for the size, then with it.
 struct Carver {

@@ -293,7 +293,7 @@ struct KnnArgs {
 // Bound: instruction issue, about 200 candidates and 70 x 70 compared distances a query. N = 10^6, k = 50:
 // 1.14 ms; a query per thread with a sorted list of k+1 in LDS (four waves per CU, 130 insertions of
 // 25 moves each) took 11.3 ms. The grid kernels take 0.2 ms; binning on the host, with its copies,
-// took 27 ms of a call of 41-50 ms, which now takes 2.6 ms.
+// took 27 ms of a call of 41-50 ms, which now takes 2.2 ms.
 __global__ void __launch_bounds__(64 * KNN_WAVES) knn_grid_kernel(KnnArgs a) {
     __shared__ double s_d[KNN_WAVES][KNN_CAP];
     __shared__ int s_id[KNN_WAVES][KNN_CAP];
@@ -446,10 +446,9 @@ __global__ void __launch_bounds__(256) knn_put_rows_kernel(const int32_t* __rest
 }
 
 struct DevBuf {
+    rbfx_ctx* ctx;
     void* p = nullptr;
-    ~DevBuf() {
-        if (p) hipFree(p);
-    }
+    ~DevBuf() { rbfx_pool_free(ctx, p); }
 };
 
 unsigned blocks_for(size_t n, size_t per) { return (unsigned)((n + per - 1) / per); }
@@ -469,8 +468,8 @@ int knn_gpu_impl(rbfx_ctx* ctx, int32_t n_nodes, const double* xyz, int32_t k, i
         rows.resize(m * ((size_t)k + 1));  // the rows, then their lists
         int rc = rbfx_knn_kdtree_rows(n_nodes, xyz, k, rows.data(), (int32_t)m, rows.data() + m, 1);
         if (rc != RBFX_OK) return rc;
-        DevBuf put;
-        if (hipMalloc(&put.p, rows.size() * sizeof(int32_t)) != hipSuccess)
+        DevBuf put{ctx};
+        if (rbfx_pool_alloc(ctx, &put.p, rows.size() * sizeof(int32_t)) != hipSuccess)
             return rbfx_fail(ctx, RBFX_E_NOMEM, "knn_gpu: rows from the host");
         RBFX_HIP_CHECK(ctx, hipMemcpyAsync(put.p, rows.data(), rows.size() * sizeof(int32_t), hipMemcpyHostToDevice, st));
         knn_put_rows_kernel<<<blocks_for(m * k, 256), 256, 0, st>>>((int32_t*)put.p, (int32_t*)put.p + m, (int)m, k, d_out);
@@ -507,8 +506,8 @@ int knn_gpu_impl(rbfx_ctx* ctx, int32_t n_nodes, const double* xyz, int32_t k, i
     };
     Carver m;
     carve(m);
-    DevBuf mem;
-    hipError_t e = hipMalloc(&mem.p, m.used);
+    DevBuf mem{ctx};
+    hipError_t e = rbfx_pool_alloc(ctx, &mem.p, m.used);
     if (e != hipSuccess) return rbfx_fail(ctx, RBFX_E_NOMEM, "knn_gpu: %s", hipGetErrorString(e));
     m = Carver{(unsigned char*)mem.p};
     carve(m);

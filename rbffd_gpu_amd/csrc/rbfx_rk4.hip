@@ -414,8 +414,8 @@ int rbfx_rk4_create(rbfx_ctx* ctx, const rbfx_rk4_desc* d, rbfx_rk4** out) {
     size_t nf = (size_t)e->n_rows * rk->F;
     size_t xs = nf * (rk->field_storage == RBFX_F64 ? sizeof(double) : sizeof(float));
     hipError_t err;
-    if ((err = hipMalloc(&rk->u, nf * sizeof(double))) != hipSuccess || (err = hipMalloc(&rk->acc, nf * sizeof(double))) != hipSuccess ||
-        (err = hipMalloc(&rk->xa, xs)) != hipSuccess || (err = hipMalloc(&rk->xb, xs)) != hipSuccess) {
+    if ((err = rbfx_malloc(ctx, (void**)&rk->u, nf * sizeof(double))) != hipSuccess || (err = rbfx_malloc(ctx, (void**)&rk->acc, nf * sizeof(double))) != hipSuccess ||
+        (err = rbfx_malloc(ctx, &rk->xa, xs)) != hipSuccess || (err = rbfx_malloc(ctx, &rk->xb, xs)) != hipSuccess) {
         rbfx_rk4_destroy(rk);
         return rbfx_fail(ctx, RBFX_E_NOMEM, "rk4_create: allocation failed: %s", hipGetErrorString(err));
     }

@@ -643,7 +643,7 @@ namespace {
 void stokes_free(rbfx_stokes* S) {
     for (void* p : {S->rows_mem, S->sweep_mem, S->V, S->w, (void*)S->r64, (void*)S->x32d, (void*)S->partial,
                     (void*)S->hbuf, (void*)S->coef})
-        if (p) hipFree(p);
+        rbfx_pool_free(S->ctx, p);
 }
 
 // One sweep's order on the host: rows level by level, each row's task and chunk, and the chunks
@@ -773,24 +773,26 @@ int workspace(rbfx_stokes* S, int m) {
     if (S->ws_m >= m) return RBFX_OK;
     for (void** p : {&S->V, &S->w, (void**)&S->r64, (void**)&S->x32d, (void**)&S->coef})
         if (*p) {
-            hipFree(*p);
+            rbfx_pool_free(S->ctx, *p);
             *p = nullptr;
         }
+    S->ws_m = -1;
     const size_t n = S->n_tot;
-    bool ok = hipMalloc(&S->V, (size_t)(m + 1) * n * sizeof(double)) == hipSuccess &&
-              hipMalloc(&S->w, n * sizeof(double)) == hipSuccess && hipMalloc(&S->r64, n * sizeof(double)) == hipSuccess &&
-              hipMalloc(&S->x32d, n * sizeof(double)) == hipSuccess &&
-              hipMalloc(&S->coef, (size_t)(m + 1) * sizeof(double)) == hipSuccess;
+    bool ok = rbfx_pool_alloc(S->ctx, &S->V, (size_t)(m + 1) * n * sizeof(double)) == hipSuccess &&
+              rbfx_pool_alloc(S->ctx, &S->w, n * sizeof(double)) == hipSuccess &&
+              rbfx_pool_alloc(S->ctx, &S->r64, n * sizeof(double)) == hipSuccess &&
+              rbfx_pool_alloc(S->ctx, &S->x32d, n * sizeof(double)) == hipSuccess &&
+              rbfx_pool_alloc(S->ctx, &S->coef, (size_t)(m + 1) * sizeof(double)) == hipSuccess;
     if (!ok) {
         S->ws_m = -1;
         return rbfx_fail(S->ctx, RBFX_E_NOMEM, "stokes_gmres: workspace for Krylov dimension %d", m);
     }
-    if (S->partial) hipFree(S->partial);
-    if (S->hbuf) hipFree(S->hbuf);
+    rbfx_pool_free(S->ctx, S->partial);
+    rbfx_pool_free(S->ctx, S->hbuf);
     S->partial = nullptr;
     S->hbuf = nullptr;
-    if (hipMalloc((void**)&S->partial, (size_t)(m + 4) * DOT_BLOCKS * sizeof(double)) != hipSuccess ||
-        hipMalloc((void**)&S->hbuf, (size_t)2 * (m + 2) * sizeof(double)) != hipSuccess) {
+    if (rbfx_pool_alloc(S->ctx, &S->partial, (size_t)(m + 4) * DOT_BLOCKS * sizeof(double)) != hipSuccess ||
+        rbfx_pool_alloc(S->ctx, &S->hbuf, (size_t)2 * (m + 2) * sizeof(double)) != hipSuccess) {
         S->ws_m = -1;
         return rbfx_fail(S->ctx, RBFX_E_NOMEM, "stokes_gmres: reduction buffers");
     }
@@ -951,7 +953,7 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     };
     Carver rows_mem;
     carve_rows(rows_mem);
-    hipError_t e = hipMalloc(&S->rows_mem, rows_mem.used);
+    hipError_t e = rbfx_pool_alloc(ctx, &S->rows_mem, rows_mem.used);
     if (e != hipSuccess) return fail(RBFX_E_NOMEM, "matrix and factor", e);
     rows_mem = Carver{(unsigned char*)S->rows_mem};
     carve_rows(rows_mem);
@@ -1030,7 +1032,7 @@ int rbfx_stokes_create(rbfx_ctx* ctx, rbfx_ell* ops64, rbfx_ell* ops32, double e
     };
     Carver sweep_mem;
     carve_sweeps(sweep_mem);
-    if ((e = hipMalloc(&S->sweep_mem, sweep_mem.used)) != hipSuccess) return fail(RBFX_E_NOMEM, "packed factor entries", e);
+    if ((e = rbfx_pool_alloc(ctx, &S->sweep_mem, sweep_mem.used)) != hipSuccess) return fail(RBFX_E_NOMEM, "packed factor entries", e);
     sweep_mem = Carver{(unsigned char*)S->sweep_mem};
     carve_sweeps(sweep_mem);
     const int rc = workspace(S, 1);

@@ -2018,11 +2018,11 @@ extern "C" int rbfx_weights(rbfx_ctx* ctx, int32_t n_stencils, const int32_t* d_
     if (rc) return rc;
     RBFX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
     void* d_scratch = nullptr;
-    hipError_t e = hipMalloc(&d_scratch, wscratch_bytes(n_stencils));
+    hipError_t e = rbfx_pool_alloc(ctx, &d_scratch, wscratch_bytes(n_stencils));
     if (e != hipSuccess) return rbfx_fail(ctx, RBFX_E_NOMEM, "weights: %s", hipGetErrorString(e));
     rc = weights_impl(ctx, n_stencils, d_st_off, d_st_idx, n_nodes, d_xyz, d_eps, dertypes, dim, poly_deg, hv_k, hv_scale, mode,
                       d_w, d_diag, n_singular, d_scratch);
     hipStreamSynchronize(ctx->stream);
-    hipFree(d_scratch);
+    rbfx_pool_free(ctx, d_scratch);
     return rc;
 }
