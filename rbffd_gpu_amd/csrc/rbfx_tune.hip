@@ -66,34 +66,45 @@ EllTune default_shape(const rbfx_ell* e, int F, int ft, int acc, int kind) {
     if (F == 1 && e->n_ops <= 4 && e->width >= 24 && n <= 128ll * cus * (f64 || e->n_ops == 1 ? 1 : 2) &&
         (e->n_ops > 1 || e->width <= 64))
         return EllTune{1, 64, 8, 6};
-    // Otherwise: as many fields per thread, up to 4, as leave a wave per SIMD, for FP32 applies one per two
-    // (16 FP64 or 32 FP32 sums at most): fewer loads of the indices and weights, fewer threads. 80,000 rows x 4
-    // fields: 106 us with 4 against 112 with 2; 4096 x 4: 22 with 1 against 46 with 4; FP32: 400,000 x 8 449 with
-    // 4 against 544 with 8, 20,000 x 8 32.5 with 2 against 36.2 with 4, but 30,000 x 8 7.1 an apply with 4, 8.0 with 2.
     const int max_acc = acc == RBFX_F64 ? 16 : 32;
-    int fpt = 1;
-    for (int c : {4, 2})
-        if (F % c == 0 && c * e->n_ops <= max_acc && n * (F / c) >= (f64 || kind == 1 ? 256ll : 128ll) * cus) {
-            fpt = c;
-            break;
-        }
-    // 64-thread blocks spread few rows over more CUs (4096 rows: 22 against 29 us), 256-thread ones keep
-    // neighbouring rows of many on one CU (400,000 rows x 2: 563 against 565, 316 against 320).
-    int block = n * (F / fpt) < 1024ll * cus ? 64 : 256;
-    // A row's fields stay in one block: rows of more lanes than it has take 256-thread blocks, and beyond
-    // 256 lanes the most fields per thread, so that every field count up to 256 * 8 that divides finds a shape.
-    if (F / fpt > block) block = 256;
-    for (int c : {8, 4, 2})
-        if (F / fpt > block && F % c == 0 && c * e->n_ops <= max_acc) fpt = c;
-    // Slots per memory round trip: 16 for a single operator on one field (111 against 120 us with 4 at a
-    // million rows), else 8 (4096 rows: 22 against 25), but 4 where 8 slots of FP64 weights leave few waves:
-    // four fields on small blocks (80,000 rows x 4: 106 against more than 112; 400,000 x 8: 788 with 8, 835 with
-    // 4), applies of several operators (100,000 rows, 2: 17.8 against 18.5; 60,000 x 4 fields, 3: 12.4 with 256-thread
-    // blocks against 14.3).
-    int ub = 8;
-    if (kind == 0 && F == 1 && e->n_ops == 1) ub = 16;
-    else if (fpt == 8 || (f64 && block == 64 && (kind == 0 || fpt == 4))) ub = 4;
-    if (kind == 0 && f64 && fpt > 1) block = 256;
+    int fpt = 1, block, ub = 8;
+    if (F == 1) {
+        // 64-thread blocks spread few rows over more CUs (4096 rows: 22 against 29 us), 256-thread ones keep
+        // neighbouring rows of many on one CU. Slots per memory round trip: 16 for a single operator (111
+        // against 120 us with 4 at a million rows), else 8 (4096 rows: 22 against 25), but 4 where 8 slots of
+        // FP64 weights leave few waves (an apply of two operators, 100,000 rows: 17.8 against 18.5).
+        block = n < 1024ll * cus ? 64 : 256;
+        if (kind == 0 && e->n_ops == 1) ub = 16;
+        else if (kind == 0 && f64 && block == 64) ub = 4;
+    } else {
+        // Several fields: up to 4 per thread (16 FP64 or 32 FP32 sums at most), fewer loads of the indices
+        // and weights, as long as there is a lane for each SIMD's wave with 4, and for three waves in eight
+        // SIMDs with 2. Applies and stages, FP32 and FP64 have the line at the same place (8 fields, n = 17 to
+        // 101: at 20,000 rows 2 ahead of 4 by 2-5%, at 40,000 4 ahead of 2 by 10-18%; 4 fields: at 20,000
+        // 2 ahead of 1 by 2-14%, at 10,000 equal). Four FP64 fields in one lane lose to two lanes of two: 320,000
+        // rows x 4, n = 50, 3 operators: 542-616 us a step against 522.
+        for (int c : {4, 2})
+            if (F % c == 0 && c * e->n_ops <= max_acc && n * (F / c) >= (c == 4 ? 256ll : 96ll) * cus &&
+                !(f64 && c == 4 && F == 4)) {
+                fpt = c;
+                break;
+            }
+        // 64-thread blocks up to four waves per SIMD (40,000 rows x 5: 13% ahead; 320,000 x 3: 2-5%
+        // behind), for three FP64 fields up to one (80,000 rows: 2% behind).
+        block = n * (F / fpt) < (f64 && fpt == 1 && F == 3 ? 256ll : 1024ll) * cus ? 64 : 256;
+        // 8 slots per round trip (4: 5-15% behind), but 4 for four FP64 fields of several operators, where
+        // 8 leave few waves (80,000 rows x 8: 3-4% ahead), and for odd fields on short stencils (20,000
+        // rows x 3, n = 17, FP64: 5.5 against 6.0 us an apply).
+        if ((f64 && fpt == 4 && e->n_ops >= 3) || (fpt == 1 && F > 2 && e->width < 24 && n * F >= 192ll * cus)) ub = 4;
+        // A row's fields stay in one block: rows of more lanes than it has take 256-thread blocks, and beyond
+        // 256 lanes the most fields per thread, so that every field count up to 256 * 8 that divides finds a shape.
+        if (F / fpt > block) block = 256;
+        for (int c : {8, 4, 2})
+            if (F / fpt > block && F % c == 0 && c * e->n_ops <= max_acc) {
+                fpt = c;
+                ub = 4;
+            }
+    }
     return EllTune{fpt, block, ub, 0};
 }
 }  // namespace
