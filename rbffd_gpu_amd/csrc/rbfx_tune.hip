@@ -68,12 +68,20 @@ EllTune default_shape(const rbfx_ell* e, int F, int ft, int acc, int kind) {
         return EllTune{1, 64, 8, 6};
     const int max_acc = acc == RBFX_F64 ? 16 : 32;
     int fpt = 1, block, ub = 8;
+    // 256-thread blocks keep neighbouring rows on one CU, 64-thread ones spread the last round of blocks over
+    // all CUs: up to four waves per SIMD 64, unless 256-thread blocks fill at least 4/5 of their last round. One
+    // field, rounds of 65,536 rows: 126,000 rows (1.92 rounds) 2-5% for 256, 250,000 (3.8) 0-4%; 70,000 (1.07) 19-42%
+    // for 64, 100,000 (1.53) 4-6%, 160,000 (2.44) and 200,000 (3.05) 5-9%. 4096 rows: 22 against 29 us a step;
+    // 320,000 rows x 3: 2-5% for 256.
+    auto block_for = [&](long long lanes) {
+        const long long round = 256ll * cus;
+        return lanes >= 4 * round || (lanes > round && lanes % round * 5 >= round * 4) ? 256 : 64;
+    };
     if (F == 1) {
-        // 64-thread blocks spread few rows over more CUs (4096 rows: 22 against 29 us), 256-thread ones keep
-        // neighbouring rows of many on one CU. Slots per memory round trip: 16 for a single operator (111
-        // against 120 us with 4 at a million rows), else 8 (4096 rows: 22 against 25), but 4 where 8 slots of
-        // FP64 weights leave few waves (an apply of two operators, 100,000 rows: 17.8 against 18.5).
-        block = n < 1024ll * cus ? 64 : 256;
+        // Slots per memory round trip: 16 for a single operator (111 against 120 us with 4 at a million rows),
+        // else 8 (4096 rows: 22 against 25), but 4 where 8 slots of FP64 weights leave few waves (an apply
+        // of two operators, 100,000 rows: 17.8 against 18.5).
+        block = block_for(n);
         if (kind == 0 && e->n_ops == 1) ub = 16;
         else if (kind == 0 && f64 && block == 64) ub = 4;
     } else {
@@ -89,9 +97,7 @@ EllTune default_shape(const rbfx_ell* e, int F, int ft, int acc, int kind) {
                 fpt = c;
                 break;
             }
-        // 64-thread blocks up to four waves per SIMD (40,000 rows x 5: 13% ahead; 320,000 x 3: 2-5%
-        // behind), for three FP64 fields up to one (80,000 rows: 2% behind).
-        block = n * (F / fpt) < (f64 && fpt == 1 && F == 3 ? 256ll : 1024ll) * cus ? 64 : 256;
+        block = block_for(n * (F / fpt));
         // 8 slots per round trip (4: 5-15% behind), but 4 for four FP64 fields of several operators, where
         // 8 leave few waves (80,000 rows x 8: 3-4% ahead), and for odd fields on short stencils (20,000
         // rows x 3, n = 17, FP64: 5.5 against 6.0 us an apply).
