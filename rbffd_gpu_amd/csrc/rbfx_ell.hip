@@ -29,9 +29,10 @@ struct WPtrs {
 // at most PACK_SLOTS (one chunk up to n = 128), operators in groups of PACK_OPS; R is what keeps
 // the block's LDS below 32 KB (five blocks per CU; n = 50, 4 operators: 16 rows).
 // Bound: memory (8 bytes read per weight), with one wave of four busy while a block rounds.
-// 400,009 rows, n = 50, 4 operators, FP32 with row sums: 0.56 ms (2.0 TB/s); one thread per entry
-// and another kernel for the sums took 1.02 + 2.34 ms. 8 or 32 rows per block: 0.65 and 0.68 ms,
-// 512 threads: 0.61 ms.
+// 400,009 rows, n = 50, 4 operators, FP32 with row sums: 0.51 ms (2.2 TB/s); with slots read one by one while
+// rounding, and divisions by R, 0.55; one thread per entry and another kernel for the sums 1.02 +
+// 2.34 ms. 8 or 32 rows per block: 0.65 and 0.68 ms, 512 threads: 0.61 ms, all operators' loads in
+// one loop with stepped instead of divided places: 0.62 ms.
 //
 // SUM (FP32 storage, row sums preserved): round each weight to nearest, then walk the slots in
 // stencil order (centre first, then by distance, which is roughly descending magnitude) and
@@ -71,13 +72,13 @@ __global__ void __launch_bounds__(PACK_THREADS) ell_pack_kernel(const int32_t* _
     const int S = C | 1;  // row stride in LDS: odd, so that rows start in different banks
     double* sw = reinterpret_cast<double*>(smem);                       // [op][row][slot]
     int32_t* si = reinterpret_cast<int32_t*>(sw + (size_t)PACK_OPS * R * S);  // [row][slot]
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, rs = __ffs(R) - 1;  // R is a power of two
     const int r0 = blockIdx.x * R;
     const int nr = max(0, min(R, n_rows - r0));  // rows past the end: index 0, weight 0
     const size_t dst0 = ell_row_base(r0, width);  // R divides ELL_TILE: the rows share a tile
     for (int g = 0; g < n_ops; g += PACK_OPS) {
         const int og = min(PACK_OPS, n_ops - g);
-        const int q = t / R, rq = t % R;  // the weights this thread rounds: operator g + q, row rq
+        const int q = t >> rs, rq = t & (R - 1);  // the weights this thread rounds: operator g + q, row rq
         const bool rounds = SUM && q < og && rq < nr;
         double s64 = 0.0, s32 = 0.0, rest = 0.0;
         // SUM needs the row sums before the first weight is rounded: a pass over the chunks for
@@ -104,22 +105,36 @@ __global__ void __launch_bounds__(PACK_THREADS) ell_pack_kernel(const int32_t* _
                 __syncthreads();
                 if (rounds) {
                     double* row = sw + ((size_t)q * R + rq) * S;
+                    // 8 slots are read from LDS together: one after the other each waits out its latency
                     if (pass == 0) {
-                        for (int j = 0; j < c; j++) {
-                            const double v = row[j];
-                            s64 += v;
-                            s32 += (double)(float)v;
+                        for (int b = 0; b < c; b += 8) {
+                            double v[8];
+#pragma unroll
+                            for (int u = 0; u < 8; u++) v[u] = row[min(b + u, c - 1)];
+#pragma unroll
+                            for (int u = 0; u < 8; u++)
+                                if (b + u < c) {
+                                    s64 += v[u];
+                                    s32 += (double)(float)v[u];
+                                }
                         }
                         rest = s64 - s32;
                     }
                     if (store)
-                        for (int j = 0; j < c; j++) row[j] = (double)round_toward_sum(row[j], rest);
+                        for (int b = 0; b < c; b += 8) {
+                            double v[8];
+#pragma unroll
+                            for (int u = 0; u < 8; u++) v[u] = row[min(b + u, c - 1)];
+#pragma unroll
+                            for (int u = 0; u < 8; u++)
+                                if (b + u < c) row[b + u] = (double)round_toward_sum(v[u], rest);
+                        }
                 }
                 if (SUM) __syncthreads();
                 if (store) {
                     // destination order: slot, row, operator
                     for (int e = t; e < c * R; e += PACK_THREADS) {
-                        const int r = e & (R - 1), j = e / R;
+                        const int r = e & (R - 1), j = e >> rs;
                         const bool in = r < nr;
                         const size_t d = dst0 + (size_t)(j0 + j) * ELL_TILE + r;
                         const double* v = sw + (size_t)r * S + j;
