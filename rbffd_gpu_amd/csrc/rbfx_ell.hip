@@ -417,8 +417,7 @@ int check_types(rbfx_ell* e, int field_type, int accum) {
 
 }  // namespace
 
-// Fields-per-thread choice for the fused kernels. A tuned entry (see rbfx_tune.hip) wins;
-// otherwise: the largest of 8/4/2/1 dividing F with at most 16 FP64 accumulators per thread.
+// Launch shape of the fused kernels: a tuned entry wins, else the rules of default_shape (rbfx_tune.hip).
 int rbfx_ell_pick(rbfx_ell* ell, int n_fields, int field_type, int accum, int kind, EllTune* t);
 
 extern "C" {
