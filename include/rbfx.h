@@ -240,7 +240,7 @@ typedef struct rbfx_rk4_desc {
     int32_t field_storage;     /* RBFX_F64: stage fields in FP64; RBFX_F32: stored in FP32   */
     int32_t accum;             /* RBFX_F64 or RBFX_F32 accumulation of the gathers          */
     const double* d_coef[16];  /* per-operator coefficient arrays (NULL = 1), n_ops used    */
-    int32_t use_graph;         /* 1: capture a step into a hipGraph and replay it           */
+    int32_t use_graph;         /* 1: replay runs of steps of one dt from a hipGraph        */
 } rbfx_rk4_desc;
 
 int rbfx_rk4_create(rbfx_ctx* ctx, const rbfx_rk4_desc* desc, rbfx_rk4** out);

@@ -31,20 +31,25 @@ struct rbfx_rk4 {
     void* xb = nullptr;
     bool have_state = false;
     EllTune tune;
-    // captured steps: one, and GRAPH_STEPS in a row (captured when a call asks for as many)
+    double dt = 0.0;  // of the last rbfx_rk4_step
+    bool have_dt = false;
+    // GRAPH_STEPS steps in a row, captured once a call of as many comes with the dt of the call before
     struct Captured {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
         double dt = 0.0;
         int layout = -1;  // operator-set layout version it was captured with
-    } one, many;
+    } steps;
 };
 
 namespace {
 
-// Steps of one replay where a call asks for at least as many: a replay costs about 4 us between its
-// first kernel and the stream's last. 20 steps of 4096 rows: 373 us with 4, 378 with 8, 373 with 16, 450
-// with 1; a stepper's first call, captures included, 452, 487, 560 and 520 us.
+// Steps of one replay where a call asks for at least as many; fewer, and those left over, are launched one by one. A
+// replay takes about 4 us between its first kernel and the stream's last: 20 steps of 4096 rows: 373 us with 4, 378
+// with 8, 373 with 16. Launched one by one they take 380 us and more of the host (41 us per 4 steps, a
+// replay 24); a single step 30 us, replayed from a graph of its own 34 to 41 (20 us of the host against 10).
+// A capture of 4 steps takes the host about 50 us, which a call with a new dt, or the only one of its stepper, would
+// pay for nothing: 4 steps of 4096 rows with a new dt in every call took 140 us, now 96.
 constexpr int GRAPH_STEPS = 4;
 
 struct StageArgs {
@@ -364,13 +369,18 @@ void drop(rbfx_rk4::Captured& c) {
     c = rbfx_rk4::Captured();
 }
 
-int capture_steps(rbfx_rk4* rk, double dt, int n_steps, rbfx_rk4::Captured& c) {
+int launch_step(rbfx_rk4* rk, double dt) {
+    int rc = RBFX_OK;
+    for (int s = 1; s <= 4 && rc == RBFX_OK; s++) rc = launch_stage(rk, s, dt);
+    return rc;
+}
+
+int capture_steps(rbfx_rk4* rk, double dt, rbfx_rk4::Captured& c) {
     rbfx_ctx* ctx = rk->ctx;
     drop(c);
     RBFX_HIP_CHECK(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     int rc = RBFX_OK;
-    for (int i = 0; i < n_steps && rc == RBFX_OK; i++)
-        for (int s = 1; s <= 4 && rc == RBFX_OK; s++) rc = launch_stage(rk, s, dt);
+    for (int i = 0; i < GRAPH_STEPS && rc == RBFX_OK; i++) rc = launch_step(rk, dt);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(ctx->stream, &g);
     if (rc != RBFX_OK) { if (g) hipGraphDestroy(g); return rc; }
@@ -427,8 +437,7 @@ void rbfx_rk4_destroy(rbfx_rk4* rk) {
     if (!rk) return;
     hipSetDevice(rk->ctx->device);
     hipStreamSynchronize(rk->ctx->stream);
-    drop(rk->one);
-    drop(rk->many);
+    drop(rk->steps);
     hipFree(rk->u);
     hipFree(rk->acc);
     hipFree(rk->xa);
@@ -467,29 +476,23 @@ int rbfx_rk4_step(rbfx_rk4* rk, double dt, int32_t n_steps) {
     bool shape_changed = (t.fpt != rk->tune.fpt || t.block != rk->tune.block || t.ub != rk->tune.ub ||
                           t.share != rk->tune.share);
     rk->tune = t;
-    if (rk->use_graph) {
-        if (shape_changed) {
-            drop(rk->one);
-            drop(rk->many);
-        }
-        for (int left = n_steps; left > 0;) {
-            const int k = left >= GRAPH_STEPS ? GRAPH_STEPS : 1;
-            rbfx_rk4::Captured& c = k > 1 ? rk->many : rk->one;
-            // the captured launches hold the operator set's buffers: recapture after a re-layout
-            if (!c.exec || c.dt != dt || c.layout != rk->ell->layout_version) {
-                int rc = capture_steps(rk, dt, k, c);
-                if (rc) return rc;
-            }
-            RBFX_HIP_CHECK(rk->ctx, hipGraphLaunch(c.exec, rk->ctx->stream));
-            left -= k;
-        }
-        return RBFX_OK;
+    if (shape_changed) drop(rk->steps);
+    // the captured launches hold the operator set's buffers: not after a re-layout
+    const bool replay = rk->steps.exec && rk->steps.dt == dt && rk->steps.layout == rk->ell->layout_version;
+    int left = n_steps;
+    for (; replay && left >= GRAPH_STEPS; left -= GRAPH_STEPS) RBFX_HIP_CHECK(rk->ctx, hipGraphLaunch(rk->steps.exec, rk->ctx->stream));
+    for (; left > 0; left--) {
+        int rc = launch_step(rk, dt);
+        if (rc) return rc;
     }
-    for (int i = 0; i < n_steps; i++)
-        for (int s = 1; s <= 4; s++) {
-            int rc = launch_stage(rk, s, dt);
-            if (rc) return rc;
-        }
+    if (n_steps < GRAPH_STEPS) return RBFX_OK;
+    const bool again = rk->have_dt && rk->dt == dt;
+    rk->dt = dt;
+    rk->have_dt = true;
+    if (rk->use_graph && again && !replay) {  // while the device works on the steps
+        const int rc = capture_steps(rk, dt, rk->steps);
+        if (rc) return rc;
+    }
     return RBFX_OK;
 }
 
