@@ -85,6 +85,12 @@ int rbfx_device_info(rbfx_ctx* ctx, char* name, int32_t name_len, int32_t* n_cu,
 /* ---- device memory helpers (the ctx's stream; host pointers are pageable) ------------ */
 int rbfx_dev_alloc(rbfx_ctx* ctx, uint64_t bytes, void** d_ptr);
 int rbfx_dev_free(rbfx_ctx* ctx, void* d_ptr);
+/* Device memory of dropped operator sets, tile tables, Stokes solvers and of the searches' and
+ * weights' scratch stays with the context for the next of them: at most 1/64 of the device's
+ * memory, in at most 32 blocks. It is given back with the context, or when an allocation of any
+ * context of this process on the device fails; this call gives it back at once, for other
+ * allocators (bytes, optional: how much). */
+int rbfx_release_idle(rbfx_ctx* ctx, uint64_t* bytes);
 int rbfx_h2d(rbfx_ctx* ctx, void* d_dst, const void* h_src, uint64_t bytes);
 int rbfx_d2h(rbfx_ctx* ctx, void* h_dst, const void* d_src, uint64_t bytes);
 int rbfx_d2d(rbfx_ctx* ctx, void* d_dst, const void* d_src, uint64_t bytes);

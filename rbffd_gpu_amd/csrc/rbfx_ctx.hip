@@ -36,9 +36,29 @@ void pool_drop_oldest(rbfx_ctx* ctx) {
     ctx->idle.erase(ctx->idle.begin());
 }
 
-void pool_trim(rbfx_ctx* ctx) {
+size_t pool_trim(rbfx_ctx* ctx) {
     std::lock_guard<std::mutex> lk(ctx->pool_mu);
+    const size_t bytes = ctx->idle_bytes;
     while (!ctx->idle.empty()) pool_drop_oldest(ctx);
+    return bytes;
+}
+
+// The contexts of this process: one that runs out of memory takes back what the others on its device keep.
+struct Contexts {
+    std::mutex mu;
+    std::vector<rbfx_ctx*> all;
+};
+
+Contexts& contexts() {
+    static Contexts* c = new Contexts();
+    return *c;
+}
+
+void trim_device(int device) {
+    Contexts& c = contexts();
+    std::lock_guard<std::mutex> lk(c.mu);
+    for (rbfx_ctx* x : c.all)
+        if (x->device == device) pool_trim(x);
 }
 }  // namespace
 
@@ -47,7 +67,7 @@ hipError_t rbfx_malloc(rbfx_ctx* ctx, void** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        pool_trim(ctx);
+        trim_device(ctx->device);
         e = hipMalloc(p, bytes);
         if (e != hipSuccess) {
             (void)hipGetLastError();
@@ -130,6 +150,10 @@ int rbfx_create(int device_ordinal, rbfx_ctx** out) {
         delete c;
         return rbfx_fail(nullptr, RBFX_E_HIP, "rbfx_create: %s", hipGetErrorString(e));
     }
+    {
+        std::lock_guard<std::mutex> lk(contexts().mu);
+        contexts().all.push_back(c);
+    }
     *out = c;
     return RBFX_OK;
 }
@@ -138,6 +162,11 @@ void rbfx_destroy(rbfx_ctx* ctx) {
     if (!ctx) return;
     hipSetDevice(ctx->device);
     hipStreamSynchronize(ctx->stream);
+    {
+        std::lock_guard<std::mutex> lk(contexts().mu);
+        auto& all = contexts().all;
+        all.erase(std::remove(all.begin(), all.end(), ctx), all.end());
+    }
     pool_trim(ctx);
     hipEventDestroy(ctx->t0);
     hipEventDestroy(ctx->t1);
@@ -167,6 +196,14 @@ int rbfx_dev_alloc(rbfx_ctx* ctx, uint64_t bytes, void** d_ptr) {
     if (bytes == 0) return RBFX_OK;
     hipError_t e = rbfx_malloc(ctx, d_ptr, bytes);
     if (e != hipSuccess) return rbfx_fail(ctx, RBFX_E_NOMEM, "hipMalloc(%llu): %s", (unsigned long long)bytes, hipGetErrorString(e));
+    return RBFX_OK;
+}
+
+int rbfx_release_idle(rbfx_ctx* ctx, uint64_t* bytes) {
+    if (!ctx) return RBFX_E_INVALID;
+    RBFX_HIP_CHECK(ctx, hipSetDevice(ctx->device));
+    const size_t b = pool_trim(ctx);
+    if (bytes) *bytes = b;
     return RBFX_OK;
 }
 

@@ -65,7 +65,7 @@ int rbfx_fail(rbfx_ctx* ctx, int code, const char* fmt, ...);
                              hipGetErrorString(e_));                                          \
     } while (0)
 
-// hipMalloc that, when memory runs out, gives the context's idle blocks back and tries again.
+// hipMalloc that, when memory runs out, gives the idle blocks of the device's contexts back and tries again.
 hipError_t rbfx_malloc(rbfx_ctx* ctx, void** p, size_t bytes);
 
 // Device memory of objects that are built and dropped again and again (operator sets, tile tables, the
@@ -73,8 +73,8 @@ hipError_t rbfx_malloc(rbfx_ctx* ctx, void** p, size_t bytes);
 // are freed and serve the next request of up to their size and at least 4/5 of it; contents are
 // whatever the last user left. Everything that touches such memory is work on the context's
 // stream, so a block's next use comes after its last one without a wait. At most 1/64 of the
-// device's memory and 32 blocks are kept; they are given back with the context, or when an
-// allocation fails.
+// device's memory and 32 blocks are kept; they are given back with the context, by
+// rbfx_release_idle, or when an allocation of any context on the device fails.
 hipError_t rbfx_pool_alloc_bytes(rbfx_ctx* ctx, void** p, size_t bytes);
 void rbfx_pool_free(rbfx_ctx* ctx, void* p);
 template <typename T>

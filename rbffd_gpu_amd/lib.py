@@ -61,6 +61,7 @@ def load_library(path=None):
         "rbfx_device_info": (C.c_int, [vp, C.c_char_p, i32, C.POINTER(i32), C.POINTER(i32)]),
         "rbfx_dev_alloc": (C.c_int, [vp, u64, C.POINTER(vp)]),
         "rbfx_dev_free": (C.c_int, [vp, vp]),
+        "rbfx_release_idle": (C.c_int, [vp, C.POINTER(u64)]),
         "rbfx_h2d": (C.c_int, [vp, vp, vp, u64]),
         "rbfx_d2h": (C.c_int, [vp, vp, vp, u64]),
         "rbfx_d2d": (C.c_int, [vp, vp, vp, u64]),
@@ -255,6 +256,12 @@ class Context:
         d = DeviceArray(self, a.shape, a.dtype)
         d.upload(a)
         return d
+
+    def release_idle(self):
+        """Gives back the device memory kept for the next objects; returns how many bytes that was."""
+        n = C.c_uint64()
+        self.check(RBFX.rbfx_release_idle(self.h, C.byref(n)))
+        return n.value
 
     def timer_start(self):
         self.check(RBFX.rbfx_timer_start(self.h))
