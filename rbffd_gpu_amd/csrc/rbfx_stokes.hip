@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "rbfx_ell_common.h"
+#include "rbfx_stokes_order.h"
 
 namespace {
 
@@ -46,9 +47,6 @@ constexpr unsigned long long FACTOR_UNSET = 0x7ff4a5a5a5a5a5a5ull;
 // registers: 12 waves of at most 168 VGPRs for the first, 8 of at most 256 for the others.
 constexpr int sweep_variant(int blks) { return blks <= 4 ? 4 : blks <= 7 ? blks : 8; }
 __host__ __device__ constexpr int sweep_waves(int nb) { return nb <= 4 ? 12 : 8; }
-constexpr int SWEEP_ROWS = 64;     // rows of a chunk, one per lane
-constexpr int SWEEP_BLK = 8;       // entries whose products a wave forms together
-constexpr int SWEEP_MAX_BLKS = 8;  // up to 64 entries of a row on one side of the diagonal
 constexpr int SWEEP_RING = 16384;  // solved values kept in LDS: the last 16384 tasks
 constexpr int SWEEP_ZERO = SWEEP_RING, SWEEP_ONE = SWEEP_RING + 1;  // LDS places holding 0 and 1
 constexpr int FACTOR_MAX_WIDTH = 64;  // one lane per stencil entry in the factorization
@@ -326,14 +324,6 @@ __global__ void factor_init_kernel(unsigned long long* f, size_t n, int* counter
 // rows, took 1.83 / 2.01 ms; this kernel with scalar loads of the entries (64 per lane and chunk, the
 // CU's load rate) 0.57 / 0.63, with the final block read ahead of the count 0.70 / 0.80, with
 // 4-entry blocks 0.96 / 1.12.
-struct SweepChunk {
-    int t0, nr;            // first task, rows
-    int base;              // first packed entry
-    int nblk;              // blocks of 8 entries; bit 8: some entries are older than the ring
-    int need[SWEEP_MAX_BLKS];  // chunks that must be done before block b's products
-    int unused[4];
-};
-
 template <typename T, bool UPPER, int NB>
 __global__ void __launch_bounds__(64 * sweep_waves(NB)) ilu0_sweep_kernel(const SweepChunk* __restrict__ chunks, int n_chunks,
                                                                      const int32_t* __restrict__ rows,
@@ -373,7 +363,7 @@ __global__ void __launch_bounds__(64 * sweep_waves(NB)) ilu0_sweep_kernel(const 
 #pragma unroll
         for (int b = 0; b < NB; b++)
             if (UPPER ? b < nblk : b >= NB - nblk) {
-                const size_t at = (size_t)C.base + (UPPER ? b : b - (NB - nblk)) * SWEEP_BLK * C.nr;
+                const size_t at = (size_t)C.base * SWEEP_BLK + (UPPER ? b : b - (NB - nblk)) * SWEEP_BLK * C.nr;
 #pragma unroll
                 for (int e = 0; e < SWEEP_BLK; e += 4) {
                     int i4[4];
@@ -553,7 +543,8 @@ __global__ void __launch_bounds__(256) pack_sweep_kernel(SweepChunk* __restrict_
                                                         double* __restrict__ dg64, float* __restrict__ dg32) {
     const int c = blockIdx.x * 4 + (int)threadIdx.x / 64, lane = threadIdx.x % 64;
     if (c >= n_chunks) return;  // uniform over the wave
-    const int t0 = chunks[c].t0, nr = chunks[c].nr, base = chunks[c].base, nblk = chunks[c].nblk;
+    const int t0 = chunks[c].t0, nr = chunks[c].nr, nblk = chunks[c].nblk;
+    const size_t base = (size_t)chunks[c].base * SWEEP_BLK;
     const bool in = lane < nr;
     const int r = rows[t0 + (in ? lane : 0)], dr = diag[r];
     const int a = upper ? dr + 1 : r * W, b = upper ? (r + 1) * W : dr;
@@ -576,9 +567,9 @@ __global__ void __launch_bounds__(256) pack_sweep_kernel(SweepChunk* __restrict_
                 }
             }
             if (in) {
-                const size_t at4 = (size_t)base + (size_t)(e / 4 * 4) * nr + 4 * lane + e % 4;
+                const size_t at4 = base + (size_t)(e / 4 * 4) * nr + 4 * lane + e % 4;
                 idx[at4] = at;
-                val64[(size_t)base + (size_t)(e / 2 * 2) * nr + 2 * lane + e % 2] = v;
+                val64[base + (size_t)(e / 2 * 2) * nr + 2 * lane + e % 2] = v;
                 if (val32) val32[at4] = (float)v;
             }
         }
@@ -644,48 +635,6 @@ void stokes_free(rbfx_stokes* S) {
     for (void* p : {S->rows_mem, S->sweep_mem, S->V, S->w, (void*)S->r64, (void*)S->x32d, (void*)S->partial,
                     (void*)S->hbuf, (void*)S->coef})
         rbfx_pool_free(S->ctx, p);
-}
-
-// One sweep's order on the host: rows level by level, each row's task and chunk, and the chunks
-// (up to SWEEP_ROWS rows of a level) with the place of their packed entries.
-struct HostSide {
-    std::vector<SweepChunk> chunks;
-    std::vector<int32_t> rows, task, chunk_of, off;
-    size_t n_ent = 0;
-};
-
-// lev[r] of n_lev levels; count(r): entries of row r on the sweep's side of the diagonal.
-template <typename Fn>
-void order_side(const std::vector<int32_t>& lev, int n_lev, const Fn& count, HostSide& D) {
-    const int N = (int)lev.size();
-    D.off.assign(n_lev + 1, 0);
-    for (int r = 0; r < N; r++) D.off[lev[r] + 1]++;
-    for (int l = 0; l < n_lev; l++) D.off[l + 1] += D.off[l];
-    D.rows.resize(N);
-    D.task.resize(N);
-    D.chunk_of.resize(N);
-    std::vector<int32_t> pos(D.off.begin(), D.off.end() - 1);
-    for (int r = 0; r < N; r++) {
-        const int t = pos[lev[r]]++;
-        D.rows[t] = r;
-        D.task[r] = t;
-    }
-    for (int l = 0; l < n_lev; l++)
-        for (int t0 = D.off[l]; t0 < D.off[l + 1]; t0 += SWEEP_ROWS) {
-            SweepChunk C = {};
-            C.t0 = t0;
-            C.nr = std::min(SWEEP_ROWS, D.off[l + 1] - t0);
-            C.base = (int)D.n_ent;
-            int most = 0;
-            for (int t = t0; t < t0 + C.nr; t++) {
-                const int r = D.rows[t];
-                most = std::max(most, count(r));
-                D.chunk_of[r] = (int)D.chunks.size();
-            }
-            C.nblk = (most + SWEEP_BLK - 1) / SWEEP_BLK;
-            D.n_ent += (size_t)C.nblk * SWEEP_BLK * C.nr;
-            D.chunks.push_back(C);
-        }
 }
 
 // The error of the stencil at layout position p, which holds a node twice or misses its centre.
