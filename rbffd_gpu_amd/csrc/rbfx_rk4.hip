@@ -31,9 +31,9 @@ struct rbfx_rk4 {
     void* xb = nullptr;
     bool have_state = false;
     EllTune tune;
-    double dt = 0.0;  // of the last rbfx_rk4_step
-    bool have_dt = false;
-    // GRAPH_STEPS steps in a row, captured once a call of as many comes with the dt of the call before
+    double dt = 0.0;  // of the last rbfx_rk4_step of GRAPH_STEPS or more
+    // GRAPH_STEPS steps in a row, captured by the first call of as many, and anew when dt (or the layout) has
+    // changed and a call comes with the dt of the call before
     struct Captured {
         hipGraph_t graph = nullptr;
         hipGraphExec_t exec = nullptr;
@@ -48,8 +48,10 @@ namespace {
 // replay takes about 4 us between its first kernel and the stream's last: 20 steps of 4096 rows: 373 us with 4, 378
 // with 8, 373 with 16. Launched one by one they take 380 us and more of the host (41 us per 4 steps, a
 // replay 24); a single step 30 us, replayed from a graph of its own 34 to 41 (20 us of the host against 10).
-// A capture of 4 steps takes the host about 50 us, which a call with a new dt, or the only one of its stepper, would
-// pay for nothing: 4 steps of 4096 rows with a new dt in every call took 140 us, now 96.
+// A capture of 4 steps takes the host about 50 us, which a call whose dt does not come again would pay for
+// nothing: 4 steps of 4096 rows with a new dt in every call took 170 to 200 us, launched one by one 86 to 96. It comes
+// before the call's own steps: graphs instantiated while the device was busy left all launches after them slower
+// (ROCm 7.2, 10^6 rows x 16 in FP32: 922 steps/s instead of 938).
 constexpr int GRAPH_STEPS = 4;
 
 struct StageArgs {
@@ -477,20 +479,21 @@ int rbfx_rk4_step(rbfx_rk4* rk, double dt, int32_t n_steps) {
                           t.share != rk->tune.share);
     rk->tune = t;
     if (shape_changed) drop(rk->steps);
-    // the captured launches hold the operator set's buffers: not after a re-layout
-    const bool replay = rk->steps.exec && rk->steps.dt == dt && rk->steps.layout == rk->ell->layout_version;
     int left = n_steps;
-    for (; replay && left >= GRAPH_STEPS; left -= GRAPH_STEPS) RBFX_HIP_CHECK(rk->ctx, hipGraphLaunch(rk->steps.exec, rk->ctx->stream));
+    if (rk->use_graph && n_steps >= GRAPH_STEPS) {
+        rbfx_rk4::Captured& c = rk->steps;
+        // the captured launches hold the operator set's buffers: not after a re-layout
+        auto current = [&] { return c.exec && c.dt == dt && c.layout == rk->ell->layout_version; };
+        if (!current() && (!c.exec || rk->dt == dt)) {
+            int rc = capture_steps(rk, dt, c);
+            if (rc) return rc;
+        }
+        rk->dt = dt;
+        if (current())
+            for (; left >= GRAPH_STEPS; left -= GRAPH_STEPS) RBFX_HIP_CHECK(rk->ctx, hipGraphLaunch(c.exec, rk->ctx->stream));
+    }
     for (; left > 0; left--) {
         int rc = launch_step(rk, dt);
-        if (rc) return rc;
-    }
-    if (n_steps < GRAPH_STEPS) return RBFX_OK;
-    const bool again = rk->have_dt && rk->dt == dt;
-    rk->dt = dt;
-    rk->have_dt = true;
-    if (rk->use_graph && again && !replay) {  // while the device works on the steps
-        const int rc = capture_steps(rk, dt, rk->steps);
         if (rc) return rc;
     }
     return RBFX_OK;
