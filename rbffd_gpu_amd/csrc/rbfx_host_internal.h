@@ -25,8 +25,8 @@ int rbfx_build_local_tables(const int32_t* idx_layout, int n_rows, int n_pad, in
 extern "C" __attribute__((visibility("hidden"))) int rbfx_knn_kdtree_rows(int32_t n_nodes, const double* xyz, int32_t k, const int32_t* rows,
                                     int32_t n_rows, int32_t* out_idx, int32_t compact);
 
-// Uniform-grid binning of the nodes on the host, the plain statement of what the GPU search does on
-// the device: bounding box corner
+// Uniform-grid binning of the nodes on the host, called by its test only (the GPU search bins on the
+// device, by a rule of its own): bounding box corner
 // lo, cell size h, cell counts g, cell start table (size g0*g1*g2 + 1) and the nodes sorted
 // by cell (coordinates pts, ids pid). RBFX_E_INVALID for non-finite coordinates.
 __attribute__((visibility("hidden"))) int rbfx_knn_grid_bin(int32_t n, const double* xyz, int32_t k, double lo[3],

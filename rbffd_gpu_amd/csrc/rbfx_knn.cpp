@@ -267,8 +267,8 @@ inline double unit_sym(uint64_t r) { return (double)(r >> 11) * (2.0 / 900719925
 
 }  // namespace
 
-// Uniform grid of cubic cells for a k-nearest-neighbour search, on the host (the GPU search bins on
-// the device, csrc/rbfx_knn_gpu.hip; this is the plain statement of such a binning): bounding
+// Uniform grid of cubic cells for a k-nearest-neighbour search, on the host. The GPU search bins on
+// the device, by a rule of its own (csrc/rbfx_knn_gpu.hip); only this function's test calls it: bounding
 // box lo..; cell size h halved from the largest extent until a non-empty cell holds about
 // (k+1)/6 nodes (at least 2) or the dense table would pass 2^25 cells; dims g; nodes sorted
 // by cell (cell index (z * gy + y) * gx + x, cell c = sorted nodes cstart[c] .. cstart[c+1],

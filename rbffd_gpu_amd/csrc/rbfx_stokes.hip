@@ -43,8 +43,11 @@ constexpr int FACTOR_BLOCKS = 256;
 constexpr int FACTOR_AHEAD = 2;       // lower entries whose values a wave asks for at once
 // What a factor entry holds until it is computed: a signalling NaN, which no operation returns.
 constexpr unsigned long long FACTOR_UNSET = 0x7ff4a5a5a5a5a5a5ull;
-// A sweep's variants hold rows of up to 32, 40, 48 or 64 entries on one side of the diagonal in
-// registers: 12 waves of at most 168 VGPRs for the first, 8 of at most 256 for the others.
+// A sweep's variants hold rows of up to 32, 40, 48, 56 or 64 entries on one side of the diagonal in
+// registers: 12 waves of at most 168 VGPRs for the first, 8 of at most 256 for the others. The longest row decides, and the
+// first and last rows of a set have n - 1 entries on one side: n = 34 and up run 8 waves. 64 entries in FP64
+// do not fit: 64 and 67 VGPRs spill, and N = 20,000 takes 2.87 ms for both sweeps at n = 58 against 1.45 at n = 57
+// (4.67 with a barrier per 32 rows).
 constexpr int sweep_variant(int blks) { return blks <= 4 ? 4 : blks <= 7 ? blks : 8; }
 __host__ __device__ constexpr int sweep_waves(int nb) { return nb <= 4 ? 12 : 8; }
 constexpr int SWEEP_RING = 16384;  // solved values kept in LDS: the last 16384 tasks

@@ -1527,7 +1527,7 @@ __device__ __attribute__((noinline)) void lu_team(const WParams& P, int start, i
     // took 79,000 cycles of an m = 111 stencil, this takes 33,000: 40,000 stencils of 101 nodes
     // 10.3 -> 9.4 ms, of 31 nodes 1.94 -> 1.70 ms, with the priorities and the shorter pivot search.
     // The loads of rows past k stay inside the team's LDS (the diagonal and the maxima follow the packed
-    // U: 15 doubles at most are read past it) and their products are not kept.
+    // U: 16 doubles at most are read past it) and their products are not kept.
     const int li = lane & 15, lq = lane >> 4;
     auto load_rhs = [&](double (&b)[RT], int t0) {
 #pragma unroll
